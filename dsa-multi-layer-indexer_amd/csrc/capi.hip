@@ -567,20 +567,11 @@ int dsa_mli_graph_destroy(dsa_mli_graph* graph) {
 int dsa_internal_debug(int on) {
   DSA_REQUIRE(!on || dsa::kPhaseStamps, DSA_ERR_INVALID_ARG,
               "dsa_internal_debug: library built without -DDSA_PHASE_STAMPS");
-  const int v = on ? 1 : 0;
-  hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(dsa::g_dbg_on), &v, sizeof(v));
-  if (e == hipSuccess && on) {
-    void* p = nullptr;
-    e = hipGetSymbolAddress(&p, HIP_SYMBOL(dsa::g_dbg));
-    if (e == hipSuccess) e = hipMemset(p, 0, sizeof(unsigned long long) * dsa::kDbgBlocks * dsa::kDbgPhases);
-  }
-  return hip_status(e, "debug enable");
+  return hip_status(dsa::debug_enable(on), "debug enable");
 }
 
 int dsa_internal_debug_read(unsigned long long* host, int n) {
-  n = std::max(0, std::min(n, dsa::kDbgBlocks * dsa::kDbgPhases));
-  return hip_status(hipMemcpyFromSymbol(host, HIP_SYMBOL(dsa::g_dbg), n * sizeof(unsigned long long)),
-                    "debug read");
+  return hip_status(dsa::debug_read(host, std::max(0, std::min(n, dsa::kDbgBlocks * dsa::kDbgPhases))), "debug read");
 }
 
 // Internal (not in the public header): selects the fp8 MFMA form of the scan.
@@ -611,6 +602,68 @@ int dsa_append_index_keys(const void* k_bf16, const int32_t* rows, const int32_t
   return hip_status(dsa::launch_append_keys(k_bf16, rows, pos, n, page_table, pt_stride, index_k, (long)num_pages,
                                             (hipStream_t)stream),
                     "append index keys");
+}
+
+size_t dsa_prefill_keys_bytes(int B, int T) { return B < 1 || T < 1 ? 0 : dsa::prefill_keys_bytes(B, T); }
+
+size_t dsa_prefill_workspace_bytes(int B, int S, int H, int T) {
+  return B < 1 || S < 1 || H < 16 || H % 16 || T < 1 ? 0 : dsa::prefill_workspace_bytes(B, S, H, T);
+}
+
+size_t dsa_selection_bits_bytes(int rows, int T) {
+  return rows < 1 || T < 1 ? 0 : (size_t)rows * dsa::selection_words(T) * sizeof(uint32_t);
+}
+
+int dsa_sparse_mla_auto_nsplit(int B, int H, int topk) {
+  return B < 1 || H < 16 || topk < 1 ? 0 : dsa::attn_auto_nsplit(topk, B, H);
+}
+
+static int check_pack(const void* kv, int dtype, int B, int T, const void* out) {
+  DSA_REQUIRE(kv && out, DSA_ERR_INVALID_ARG, "dsa_pack: null pointer");
+  DSA_REQUIRE(dtype >= 0 && dtype <= 2, DSA_ERR_INVALID_ARG, "dsa_pack: dtype must be 0 (fp32), 1 (bf16) or 2 (fp16)");
+  DSA_REQUIRE(B >= 1 && T >= 1, DSA_ERR_INVALID_ARG, "dsa_pack: B and T must be >= 1 (got %d, %d)", B, T);
+  DSA_REQUIRE(aligned16(kv) && aligned16(out), DSA_ERR_INVALID_ARG, "dsa_pack: buffers must be 16-byte aligned");
+  return DSA_OK;
+}
+
+int dsa_pack_prefill_keys(const void* kv, int dtype, int B, int T, void* keys, void* stream) {
+  int rc = check_pack(kv, dtype, B, T, keys);
+  if (rc) return rc;
+  return hip_status(dsa::launch_pack_keys(kv, dtype, B, T, keys, (hipStream_t)stream), "pack prefill keys");
+}
+
+int dsa_pack_latent_rows(const void* kv, int dtype, int B, int T, int row_stride, void* rows, void* stream) {
+  int rc = check_pack(kv, dtype, B, T, rows);
+  if (rc) return rc;
+  DSA_REQUIRE(row_stride >= T, DSA_ERR_INVALID_ARG, "dsa_pack_latent_rows: row_stride %d below T %d", row_stride, T);
+  return hip_status(dsa::launch_pack_rows(kv, dtype, B, T, row_stride, rows, (hipStream_t)stream), "pack latent rows");
+}
+
+int dsa_selection_set(const void* idx, int idx_bytes, int B, int S, int n, int T, uint32_t* bits, int32_t* slots,
+                      void* stream) {
+  DSA_REQUIRE(idx && (bits != nullptr) != (slots != nullptr), DSA_ERR_INVALID_ARG,
+              "dsa_selection_set: idx and one of bits, slots");
+  DSA_REQUIRE(idx_bytes == 4 || idx_bytes == 8, DSA_ERR_INVALID_ARG, "dsa_selection_set: idx_bytes must be 4 or 8");
+  DSA_REQUIRE(B >= 1 && S >= 1 && n >= 1 && T >= 1 && (int64_t)B * S < ((int64_t)1 << 31), DSA_ERR_INVALID_ARG,
+              "dsa_selection_set: bad shape B=%d S=%d n=%d T=%d", B, S, n, T);
+  DSA_REQUIRE(T <= DSA_SELECTION_MAX_CTX && (int64_t)B * T < ((int64_t)1 << 31), DSA_ERR_UNSUPPORTED,
+              "dsa_selection_set: T %d above %d, or B*T >= 2^31", T, DSA_SELECTION_MAX_CTX);
+  return hip_status(dsa::launch_selection_set(idx, idx_bytes == 8, B * S, n, S, T, bits, slots, (hipStream_t)stream),
+                    "selection set");
+}
+
+int dsa_prefill_attention(const void* q_bf16, const void* keys, const uint32_t* bits, void* workspace, void* out_bf16,
+                          int B, int S, int H, int T, float sm_scale, void* stream) {
+  DSA_REQUIRE(q_bf16 && keys && workspace && out_bf16, DSA_ERR_INVALID_ARG, "dsa_prefill_attention: null pointer");
+  DSA_REQUIRE(B >= 1 && S >= 1 && T >= 1 && (int64_t)B * S <= 65535, DSA_ERR_INVALID_ARG,
+              "dsa_prefill_attention: bad B*S %lld or T %d", (long long)B * S, T);
+  DSA_REQUIRE(H >= 16 && H % 16 == 0 && H <= 16 * 64, DSA_ERR_UNSUPPORTED,
+              "dsa_prefill_attention: H must be a positive multiple of 16 (got %d)", H);
+  DSA_REQUIRE(aligned16(q_bf16) && aligned16(keys) && aligned16(workspace) && aligned16(out_bf16),
+              DSA_ERR_INVALID_ARG, "dsa_prefill_attention: buffers must be 16-byte aligned");
+  return hip_status(dsa::launch_prefill_attention(q_bf16, keys, bits, workspace, out_bf16, B, S, H, T, sm_scale,
+                                                  (hipStream_t)stream),
+                    "prefill attention");
 }
 
 int dsa_append_latent_rows(const void* latent_bf16, const int32_t* slots, int n, void* kv_pool, int64_t kv_rows,

@@ -1933,6 +1933,20 @@ int group_wait_timeouts(int reset) {
   return v;
 }
 
+hipError_t debug_enable(int on) {
+  const int v = on ? 1 : 0;
+  hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(g_dbg_on), &v, sizeof(v));
+  if (e == hipSuccess && on) {
+    void* p = nullptr;
+    e = hipGetSymbolAddress(&p, HIP_SYMBOL(g_dbg));
+    if (e == hipSuccess) e = hipMemset(p, 0, sizeof(unsigned long long) * kDbgBlocks * kDbgPhases);
+  }
+  return e;
+}
+hipError_t debug_read(unsigned long long* host, int n) {
+  return hipMemcpyFromSymbol(host, HIP_SYMBOL(g_dbg), n * sizeof(unsigned long long));
+}
+
 void set_spin_limit(int n) {
   const int v = n < 0 ? kGroupSpinMax : n;
   (void)hipMemcpyToSymbol(HIP_SYMBOL(g_group_spin_max), &v, sizeof(int));

@@ -293,6 +293,7 @@ __device__ __forceinline__ void wait_expired(uint32_t* status) {
   atomicAdd(status, 1u);
 }
 constexpr int kGroupSyncGroups = 16, kGroupSyncFlags = 8, kGroupSyncLine = 64;
+constexpr int kSyncWords = (kGroupSyncGroups + 1 + kGroupSyncFlags) * kGroupSyncLine;  // one barrier area
 constexpr int kGroupFlatMax = 32;  // groups up to this size use one arrival counter
 __device__ __forceinline__ uint32_t group_sense(const uint32_t* sync, int bid) {
   return __hip_atomic_load(&sync[(kGroupSyncGroups + 1 + (bid & (kGroupSyncFlags - 1))) * kGroupSyncLine],

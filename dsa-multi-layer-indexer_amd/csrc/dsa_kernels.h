@@ -70,6 +70,8 @@ void set_flat_scan(int on);
 void set_scan_blocks_cap(int n);
 int group_wait_timeouts(int reset);
 void set_spin_limit(int n);  // < 0: the default
+hipError_t debug_enable(int on);  // phase timestamps (profiling builds)
+hipError_t debug_read(unsigned long long* host, int n);
 // Sum of the expired-wait status words of B_scan top-k scratch rows and
 // `groups` attention barrier areas (B * H/16) into *out (device int).
 hipError_t launch_sync_status(void* topk_scratch, int B_scan, int slab, void* workspace, int groups, int* out,
@@ -95,6 +97,18 @@ hipError_t launch_topk_hist(const float* scores, const int* seq_lens, void* scra
 hipError_t launch_topk_select(const float* scores, const int* seq_lens, const int* page_table,
                               int pt_stride, void* scratch, int* out, int B, int slab, int K,
                               int sorted, int pad, hipStream_t s);
+
+// Prefill attention over bf16 keys (prefill.hip).  dtype: 0 fp32, 1 bf16, 2
+// fp16; mask == nullptr: causal only.
+size_t prefill_keys_bytes(int B, int T);
+size_t prefill_workspace_bytes(int B, int S, int H, int T);
+int selection_words(int T);
+hipError_t launch_pack_keys(const void* kv, int dtype, int B, int T, void* keys, hipStream_t s);
+hipError_t launch_pack_rows(const void* kv, int dtype, int B, int T, int stride, void* rows, hipStream_t s);
+hipError_t launch_selection_set(const void* idx, int idx64, int rows, int n, int S, int T, uint32_t* bits, int* slots,
+                                hipStream_t s);
+hipError_t launch_prefill_attention(const void* q, const void* keys, const uint32_t* mask, void* workspace, void* out,
+                                    int B, int S, int H, int T, float sm_scale, hipStream_t s);
 
 // Decode-step operand preparation (quant.hip).
 hipError_t launch_quant_query(const void* q_bf16, const float* w, void* codes, float* w_out, long rows,

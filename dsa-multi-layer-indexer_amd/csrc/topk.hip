@@ -62,7 +62,6 @@ __host__ __device__ inline long bitmap_words(int slab) { return ((long)slab + 20
 constexpr int kSyncGroups = 16;
 constexpr int kSyncFlags = 8;
 constexpr int kSyncLine = 64;  // words
-constexpr int kSyncWords = (kSyncGroups + 1 + kSyncFlags) * kSyncLine;
 constexpr int kNumSync = 4;  // slots 0 and 3: the list barrier (group_barrier_rep)
 static_assert(kSyncGroups == kGroupSyncGroups && kSyncFlags == kGroupSyncFlags && kSyncLine == kGroupSyncLine,
               "group-barrier layout");

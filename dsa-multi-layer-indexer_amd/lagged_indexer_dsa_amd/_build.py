@@ -11,6 +11,7 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -20,7 +21,7 @@ CSRC = ROOT_DIR / "csrc"
 INCLUDE = REPO_DIR / "include"
 LIB_DIR = PKG_DIR / "_lib"
 LIB_PATH = LIB_DIR / "libdsa_mli.so"
-SOURCES = ["libdsa_mli.hip"]
+SOURCES = ["libdsa_mli.hip", "capi.hip", "prefill.hip", "quant.hip", "sol.hip"]
 ARCH = "gfx950"
 
 
@@ -38,21 +39,29 @@ def build(verbose: bool = False, out: Path | None = None, phase_stamps: bool = F
     target = Path(out) if out else LIB_PATH
     target.parent.mkdir(parents=True, exist_ok=True)
     tmp = target.with_suffix(".so.tmp")
-    cmd = [
-        hipcc(), f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
+    flags = [
+        f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
         # packed fp32 VALU ops are disabled on purpose (they have produced
         # silent wrong results on this hardware pool)
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
         f"-I{INCLUDE}", f"-I{CSRC}",
         *(["-DDSA_PHASE_STAMPS"] if phase_stamps else []),
-        *[str(CSRC / s) for s in SOURCES],
-        "-o", str(tmp),
     ]
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({res.returncode}):\n{res.stderr[-4000:]}")
-    if verbose and res.stderr:
-        print(res.stderr, file=sys.stderr)
+    errs = []
+    with tempfile.TemporaryDirectory() as d:  # the sources compile side by side
+        objs = [Path(d) / (Path(s).stem + ".o") for s in SOURCES]
+        procs = [subprocess.Popen([hipcc(), *flags, "-c", str(CSRC / s), "-o", str(o)], stderr=subprocess.PIPE,
+                                  text=True) for s, o in zip(SOURCES, objs)]
+        for p in procs:
+            errs.append(p.communicate()[1])
+            if p.returncode != 0:
+                raise RuntimeError(f"hipcc failed ({p.returncode}):\n{errs[-1][-4000:]}")
+        res = subprocess.run([hipcc(), f"--offload-arch={ARCH}", "-shared", *map(str, objs), "-o", str(tmp)],
+                             capture_output=True, text=True)
+        if res.returncode != 0:
+            raise RuntimeError(f"hipcc failed ({res.returncode}):\n{res.stderr[-4000:]}")
+    if verbose:
+        print("".join(errs) + res.stderr, file=sys.stderr)
     os.replace(tmp, target)
     return target
 

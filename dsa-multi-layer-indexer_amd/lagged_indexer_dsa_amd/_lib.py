@@ -31,6 +31,7 @@ ROPE_DIM = 64
 QK_DIM = 576
 LATENT_ROW_BYTES = 656
 TOPK_MAX_CTX = 262144
+SELECTION_MAX_CTX = 524288
 
 _vp = ctypes.c_void_p
 _i32 = ctypes.c_int
@@ -88,6 +89,14 @@ SIGNATURES = {
     "dsa_quantize_index_query": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _vp]),
     "dsa_append_index_keys": (_i32, [_vp, _vp, _vp, _i32, _vp, _i32, _vp, _i64, _vp]),
     "dsa_append_latent_rows": (_i32, [_vp, _vp, _i32, _vp, _i64, _vp]),
+    "dsa_prefill_keys_bytes": (ctypes.c_size_t, [_i32, _i32]),
+    "dsa_prefill_workspace_bytes": (ctypes.c_size_t, [_i32, _i32, _i32, _i32]),
+    "dsa_selection_bits_bytes": (ctypes.c_size_t, [_i32, _i32]),
+    "dsa_sparse_mla_auto_nsplit": (_i32, [_i32, _i32, _i32]),
+    "dsa_pack_prefill_keys": (_i32, [_vp, _i32, _i32, _i32, _vp, _vp]),
+    "dsa_pack_latent_rows": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp]),
+    "dsa_selection_set": (_i32, [_vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp]),
+    "dsa_prefill_attention": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _vp]),
 }
 
 

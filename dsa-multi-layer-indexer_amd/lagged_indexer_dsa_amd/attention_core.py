@@ -20,7 +20,9 @@ implement:
   -> the sentinel ``S_kv`` (attention_core.py:66-91).
 * :func:`sparse_mla_core` quantises the latent rows to the 656-byte fp8
   format (512 e4m3 + 4 fp32 per-128 scales + 64 bf16 rope; K:1181-1197)
-  and the queries to bf16, and runs the split-K sparse MLA kernel.  A row
+  and the queries to bf16, and runs the split-K sparse MLA kernel over each
+  row's gathered keys, or the prefill kernel over all keys with the others
+  masked (the same values either way).  A row
   with no admissible key returns 0 (the GPU kernels' rule, K:1038-1042;
   the dense CPU op would return NaN there).
 
@@ -35,7 +37,7 @@ from __future__ import annotations
 import torch
 
 from . import formats, ops
-from ._lib import INDEX_DIM, LATENT_DIM, PAGE_TOKENS, QK_DIM, TOPK_MAX_CTX
+from ._lib import INDEX_DIM, LATENT_DIM, PAGE_TOKENS, QK_DIM, SELECTION_MAX_CTX, TOPK_MAX_CTX
 
 def _gpu(*ts: torch.Tensor) -> None:
     for t in ts:
@@ -117,9 +119,30 @@ def select_topk(logits: torch.Tensor, topk: int) -> torch.Tensor:
 
 def _pool_rows(kv: torch.Tensor) -> torch.Tensor:
     """[B, S_kv, 576] -> the 656-byte fp8 latent rows, batch-major slots."""
-    B, Skv, _ = kv.shape
-    flat = kv.reshape(B * Skv, QK_DIM)
-    return formats.pack_latent_rows(flat[:, :LATENT_DIM], flat[:, LATENT_DIM:]).contiguous()
+    return ops.pack_latent_rows(kv, kv.shape[1])
+
+
+def _attend_by_tiles(B: int, S: int, H: int, Skv: int, n: int) -> bool:
+    """Whether selections of n entries are attended by the prefill kernel,
+    which reads every key once per 128 (query, head) rows and masks the
+    others, or gathered row by row.
+
+    With the chip full (4096 rows and more) a gathered key costs about what
+    3.5 to 4 streamed ones do (1024 queries x 16 heads, top-2048: 4096 tokens
+    180 us against 289, 8192 tokens 312 against 298, 16384 tokens 570 against
+    310); with fewer rows the gather spreads over the idle CUs and the line
+    lies near 2 (100 queries, top-2048: 2048 tokens 45 against 52, 4096 equal,
+    8192 69 against 57); with a handful of queries both are a few launches
+    and splitting the stream over the CUs is as quick up to a few thousand
+    tokens (4 queries: 4096 tokens 33 against 43 us, 12000 tokens 44 against
+    43; 16 queries: 2048 tokens 37 against 43, 4096 tokens 45 against 43)."""
+    rows = B * S * H
+    visible = Skv - (S - 1) / 2
+    if rows <= 64:
+        return visible <= 8192
+    if rows <= 256:
+        return visible <= 4096
+    return visible <= (3.5 if rows >= 4096 else 2.0) * n
 
 
 def _attend_rows(q: torch.Tensor, kv: torch.Tensor, idx: torch.Tensor, sm_scale: float) -> torch.Tensor:
@@ -164,10 +187,21 @@ def sparse_mla_core(q: torch.Tensor, kv: torch.Tensor, indices: torch.Tensor, va
     if indices.dim() != 3 or indices.shape[:2] != q.shape[:2]:
         raise ValueError(f"indices must be [B,S,topk], got {tuple(indices.shape)}")
     _gpu(indices)
-    S, Skv = q.shape[1], kv.shape[1]
+    B, S, H, _ = q.shape
+    Skv, n = kv.shape[1], indices.shape[2]
     if sm_scale is None:
         sm_scale = q.shape[-1] ** -0.5
-    idx = indices.long()
+    idx = indices if indices.dtype in (torch.int32, torch.int64) else indices.long()
+    if 1 <= Skv <= SELECTION_MAX_CTX and B * Skv < 1 << 31 and B * S >= 1 and n >= 1:
+        if B * S <= 65535 and _attend_by_tiles(B, S, H, Skv, n):
+            out = ops.prefill_attention(q.to(torch.bfloat16).contiguous(), kv, ops.selection_set(idx, Skv, True),
+                                        float(sm_scale))
+        else:
+            qb = q.reshape(B * S, H, QK_DIM).to(torch.bfloat16).contiguous()
+            out = ops.sparse_mla_decode(qb, _pool_rows(kv), ops.selection_set(idx, Skv, False),
+                                        sm_scale=float(sm_scale))
+        return out.reshape(B, S, H, LATENT_DIM).to(q.dtype)
+    idx = idx.long()
     q_pos = _q_pos(S, Skv, q.device)[None, :, None]
     ok = (idx >= 0) & (idx < Skv) & (idx <= q_pos)
     return _attend_rows(q, kv, torch.where(ok, idx, torch.full_like(idx, -1)), float(sm_scale))
@@ -177,26 +211,19 @@ def dense_mla_core(q: torch.Tensor, kv: torch.Tensor, value_dim: int,
                    sm_scale: float | None = None) -> torch.Tensor:
     """Dense causal MLA (full-attention layers and the DENSE cold start,
     attention_core.py:142-160): query row s attends keys 0 .. S_kv - S + s,
-    on the dense MLA kernel (no limit on S_kv).  The latent rows are packed
-    to the fp8 format once, batch b's into pages of its own; every query row
-    is a decode row over its causal prefix of those pages."""
+    on the prefill kernel (no limit on S_kv), at every number of rows: down to
+    one query of 16 heads it reads and converts the keys once for all of
+    them (measured against a decode row per query: 1 query over 8192 keys 33
+    against 144 us, 8 over 1000 31 against 111, 1000 over 1000 74 against
+    194)."""
     _check_mla(q, kv, value_dim)
     B, S, H, _ = q.shape
-    Skv = kv.shape[1]
     if sm_scale is None:
         sm_scale = q.shape[-1] ** -0.5
-    dev = q.device
-    npg = max(1, (Skv + PAGE_TOKENS - 1) // PAGE_TOKENS)
-    rows = torch.zeros(B, npg * PAGE_TOKENS, QK_DIM, dtype=kv.dtype, device=dev)
-    rows[:, :Skv] = kv
-    pool = _pool_rows(rows)  # slot of (b, j) = b * npg * 64 + j
-    pt = (torch.arange(B, dtype=torch.int32, device=dev)[:, None] * npg
-          + torch.arange(npg, dtype=torch.int32, device=dev)[None, :])
-    pt_rows = pt.repeat_interleave(S, dim=0).contiguous()
-    lens = (_q_pos(S, Skv, dev) + 1).clamp(min=0).to(torch.int32).repeat(B).contiguous()
-    qb = q.reshape(B * S, H, QK_DIM).to(torch.bfloat16).contiguous()
-    out = ops.dense_mla_decode(qb, pool, pt_rows, lens, sm_scale=float(sm_scale))
-    return out.reshape(B, S, H, LATENT_DIM).to(q.dtype)
+    if kv.shape[1] == 0:  # no key: every row is empty
+        return torch.zeros(B, S, H, LATENT_DIM, dtype=q.dtype, device=q.device)
+    out = ops.prefill_attention(q.to(torch.bfloat16).contiguous(), kv, sm_scale=float(sm_scale))
+    return out.to(q.dtype)
 
 
 _NAMES = ("pad_index", "indexer_logits", "apply_causal_mask", "select_topk", "sparse_mla_core",

@@ -17,6 +17,7 @@ from ._lib import (
     INDEX_PAGE_BYTES,
     LATENT_DIM,
     LATENT_ROW_BYTES,
+    PAGE_TOKENS,
     QK_DIM,
 )
 
@@ -136,6 +137,24 @@ def sparse_mla_workspace(B: int, H: int, nsplit: int, device) -> torch.Tensor:
     return torch.zeros(nbytes // 4, dtype=torch.float32, device=device)
 
 
+def _call_workspace(B: int, H: int, nsplit: int, device) -> torch.Tensor:
+    """Workspace of one call at a known split count: the barriers zeroed, the
+    partials (overwritten before they are read) not."""
+    lib = _lib.load()
+    nbytes = lib.dsa_sparse_mla_workspace_bytes(B, H, nsplit)
+    if nbytes == 0:
+        raise RuntimeError(f"bad sparse MLA workspace shape B={B} H={H} nsplit={nsplit}")
+    ws = torch.empty(nbytes // 4, dtype=torch.float32, device=device)
+    partials = nsplit * B * (H // 16) * 16 * (LATENT_DIM + 2)
+    ws[:ws.numel() - partials].zero_()
+    return ws
+
+
+def _resolve_nsplit(nsplit: int, B: int, H: int, keys: int) -> int:
+    """The split count a call takes (nsplit = 0: the library's choice)."""
+    return nsplit or max(1, _lib.load().dsa_sparse_mla_auto_nsplit(B, H, keys))
+
+
 def sparse_mla_decode(q: torch.Tensor, kv_pool: torch.Tensor, idx: torch.Tensor,
                       sm_scale: float | None = None, nsplit: int = 0,
                       workspace: torch.Tensor | None = None,
@@ -157,7 +176,8 @@ def sparse_mla_decode(q: torch.Tensor, kv_pool: torch.Tensor, idx: torch.Tensor,
     if sm_scale is None:
         sm_scale = QK_DIM ** -0.5
     if workspace is None:
-        workspace = sparse_mla_workspace(B, H, nsplit, q.device)
+        nsplit = _resolve_nsplit(nsplit, B, H, idx.shape[1])
+        workspace = _call_workspace(B, H, nsplit, q.device)
     if out is None:
         out = torch.empty(B, H, LATENT_DIM, dtype=torch.bfloat16, device=q.device)
     _dev(workspace, out)
@@ -193,7 +213,8 @@ def dense_mla_decode(q: torch.Tensor, kv_pool: torch.Tensor, page_table: torch.T
     if sm_scale is None:
         sm_scale = QK_DIM ** -0.5
     if workspace is None:
-        workspace = sparse_mla_workspace(B, H, nsplit, q.device)
+        nsplit = _resolve_nsplit(nsplit, B, H, page_table.shape[1] * PAGE_TOKENS)
+        workspace = _call_workspace(B, H, nsplit, q.device)
     if out is None:
         out = torch.empty(B, H, LATENT_DIM, dtype=torch.bfloat16, device=q.device)
     _dev(workspace, out)
@@ -202,6 +223,75 @@ def dense_mla_decode(q: torch.Tensor, kv_pool: torch.Tensor, page_table: torch.T
     _lib.call("dsa_dense_mla_decode", q.data_ptr(), kv_pool.data_ptr(), kv_pool.shape[0], page_table.data_ptr(),
               page_table.shape[1], seq_lens.data_ptr(), workspace.data_ptr(), out.data_ptr(), B, H, nsplit,
               float(sm_scale), _stream())
+    return out
+
+
+# ---- prefill attention (many query rows against the same keys) ----
+
+_PACK_DTYPES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
+
+
+def _pack_source(kv: torch.Tensor) -> torch.Tensor:
+    """kv [B, T, 576] as the pack kernels read it: fp32, bf16 or fp16,
+    contiguous, 16-byte aligned."""
+    if kv.dtype not in _PACK_DTYPES:
+        x = kv.float()
+        x[..., LATENT_DIM:] = kv[..., LATENT_DIM:].to(torch.bfloat16)
+        kv = x
+    kv = kv.contiguous()
+    return kv if kv.data_ptr() % 16 == 0 else kv.clone()
+
+
+def pack_latent_rows(kv: torch.Tensor, row_stride: int) -> torch.Tensor:
+    """kv [B, T, 576] -> 656-byte fp8 rows [B * row_stride, 656] (rows past T
+    of a request zero)."""
+    kv = _pack_source(kv)
+    _dev(kv)
+    B, T, _ = kv.shape
+    rows = torch.empty(B * row_stride, LATENT_ROW_BYTES, dtype=torch.uint8, device=kv.device)
+    _lib.call("dsa_pack_latent_rows", kv.data_ptr(), _PACK_DTYPES[kv.dtype], B, T, row_stride, rows.data_ptr(),
+              _stream())
+    return rows
+
+
+def selection_set(idx: torch.Tensor, T: int, as_bits: bool) -> torch.Tensor:
+    """Selections idx [B, S, n] (int32 or int64 positions) as sets over the
+    row's causal keys (query row s of S sees keys 0 .. T - S + s): a bitmap per
+    row, or the KV slots b * T + position ascending, then -1 [B * S, n]."""
+    idx = idx.contiguous()
+    _dev(idx)
+    B, S, n = idx.shape
+    lib = _lib.load()
+    if as_bits:
+        out = torch.empty(lib.dsa_selection_bits_bytes(B * S, T) // 4, dtype=torch.int32, device=idx.device)
+    else:
+        out = torch.empty(B * S, n, dtype=torch.int32, device=idx.device)
+    _lib.call("dsa_selection_set", idx.data_ptr(), idx.element_size(), B, S, n, T,
+              out.data_ptr() if as_bits else None, None if as_bits else out.data_ptr(), _stream())
+    return out
+
+
+def prefill_attention(q: torch.Tensor, kv: torch.Tensor, bits: torch.Tensor | None = None,
+                      sm_scale: float | None = None) -> torch.Tensor:
+    """q [B, S, H, 576] bf16 over kv [B, T, 576]: query row s of S attends keys
+    0 .. T - S + s, or those of its bitmap (:func:`selection_set`) ->
+    [B, S, H, 512] bf16.  Reference: attention_core.py:121-160."""
+    kv = _pack_source(kv)
+    _dev(q, kv)
+    if q.dtype != torch.bfloat16:
+        raise RuntimeError("q must be bfloat16")
+    B, S, H, _ = q.shape
+    T = kv.shape[1]
+    lib = _lib.load()
+    keys = torch.empty(lib.dsa_prefill_keys_bytes(B, T), dtype=torch.uint8, device=q.device)
+    ws = torch.empty(lib.dsa_prefill_workspace_bytes(B, S, H, T), dtype=torch.uint8, device=q.device)
+    out = torch.empty(B, S, H, LATENT_DIM, dtype=torch.bfloat16, device=q.device)
+    if bits is not None:
+        _need_bytes("bits", bits, lib.dsa_selection_bits_bytes(B * S, T))
+    st = _stream()
+    _lib.call("dsa_pack_prefill_keys", kv.data_ptr(), _PACK_DTYPES[kv.dtype], B, T, keys.data_ptr(), st)
+    _lib.call("dsa_prefill_attention", q.data_ptr(), keys.data_ptr(), _ptr(bits), ws.data_ptr(), out.data_ptr(),
+              B, S, H, T, float(QK_DIM ** -0.5 if sm_scale is None else sm_scale), st)
     return out
 
 

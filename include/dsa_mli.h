@@ -53,6 +53,7 @@ extern "C" {
 #define DSA_QK_DIM 576
 #define DSA_LATENT_ROW_BYTES 656  /* 512 + 4*4 + 64*2 */
 #define DSA_TOPK_MAX_CTX 262144   /* longest row the top-k select accepts */
+#define DSA_SELECTION_MAX_CTX 524288 /* longest context of dsa_selection_set */
 
 /* dsa_topk flags */
 #define DSA_TOPK_POSITION_ORDER 0 /* selected indices ascending, pads last */
@@ -354,6 +355,39 @@ int dsa_append_index_keys(const void* k_bf16, const int32_t* rows, const int32_t
  */
 int dsa_append_latent_rows(const void* latent_bf16, const int32_t* slots, int n, void* kv_pool, int64_t kv_rows,
                            void* stream);
+
+/*
+ * (7) Prefill attention: S query rows at the end of each request's T keys.
+ * Row s of request b sees keys 0 .. T - S + s; all heads share the keys.
+ *
+ * dsa_pack_prefill_keys: kv [B, T, 576] (dtype 0 fp32, 1 bf16, 2 fp16) ->
+ *   keys, dsa_prefill_keys_bytes(B, T) bytes: the bf16 values that (3)'s
+ *   656-byte rows of the same input hold, rows padded to whole key tiles.
+ * dsa_pack_latent_rows: the 656-byte rows themselves, row_stride rows a
+ *   request (those past T zero).
+ * dsa_selection_set: idx [B, S, n] (int32 or int64 key positions, any order,
+ *   repeats and entries outside the row's keys allowed) as sets; exactly one
+ *   of bits (dsa_selection_bits_bytes(B * S, T) bytes: a bitmap a row) and
+ *   slots ([B * S, n] int32: b * T + position ascending, then -1).
+ * dsa_prefill_attention: out[b, s, h, :] as (3) over the row's keys, or over
+ *   those of its bitmap when bits is not NULL; a row without a key gives 0.
+ *   q [B, S, H, 576] bf16, out [B, S, H, 512] bf16, workspace
+ *   dsa_prefill_workspace_bytes(B, S, H, T) bytes (no initialisation);
+ *   B * S <= 65535, H a multiple of 16.
+ * dsa_sparse_mla_auto_nsplit: the split count (3) takes at nsplit = 0.
+ * Replaces: dense_mla_core and sparse_mla_core over many query rows
+ * (attention_core.py:94-160).
+ */
+size_t dsa_prefill_keys_bytes(int B, int T);
+size_t dsa_prefill_workspace_bytes(int B, int S, int H, int T);
+size_t dsa_selection_bits_bytes(int rows, int T);
+int dsa_sparse_mla_auto_nsplit(int B, int H, int topk);
+int dsa_pack_prefill_keys(const void* kv, int dtype, int B, int T, void* keys, void* stream);
+int dsa_pack_latent_rows(const void* kv, int dtype, int B, int T, int row_stride, void* rows, void* stream);
+int dsa_selection_set(const void* idx, int idx_bytes, int B, int S, int n, int T, uint32_t* bits, int32_t* slots,
+                      void* stream);
+int dsa_prefill_attention(const void* q_bf16, const void* keys, const uint32_t* bits, void* workspace, void* out_bf16,
+                          int B, int S, int H, int T, float sm_scale, void* stream);
 
 #ifdef __cplusplus
 }
