@@ -433,6 +433,9 @@ int dsa_topk(const float* scores, const int32_t* seq_lens, const int32_t* page_t
     S.pad = pad_value;
     return hip_status(dsa::launch_decode_main(nullptr, 0, &S, B, s), "top-k launch");
   }
+  if (dsa::select_rows_takes(B, slab_stride, topk))
+    return hip_status(dsa::launch_select_rows(scores, seq_lens, out_idx, 0, B, slab_stride, topk, pad_value, s),
+                      "top-k row select launch");
   rc = hip_status(dsa::launch_topk_hist(scores, seq_lens, scratch, B, slab_stride, topk, s),
                   "top-k histogram launch");
   if (rc) return rc;
@@ -440,6 +443,21 @@ int dsa_topk(const float* scores, const int32_t* seq_lens, const int32_t* page_t
                                             out_idx, B, slab_stride, topk,
                                             flags == DSA_TOPK_SORTED, pad_value, s),
                     "top-k select launch");
+}
+
+int dsa_select_rows_supported(int B, int slab_stride, int topk) {
+  return B >= 1 && B <= 65535 && topk >= 1 && slab_stride >= 1 && slab_stride <= DSA_TOPK_MAX_CTX &&
+         dsa::select_rows_takes(B, slab_stride, topk);
+}
+
+int dsa_select_rows(const float* scores, const int32_t* seq_lens, int64_t* out_idx, int B, int slab_stride, int topk,
+                    int32_t pad_value, void* stream) {
+  DSA_REQUIRE(scores && out_idx, DSA_ERR_INVALID_ARG, "dsa_select_rows: null pointer argument");
+  DSA_REQUIRE(dsa_select_rows_supported(B, slab_stride, topk), DSA_ERR_UNSUPPORTED,
+              "dsa_select_rows: B=%d slab_stride=%d topk=%d (see dsa_select_rows_supported)", B, slab_stride, topk);
+  return hip_status(dsa::launch_select_rows(scores, seq_lens, out_idx, 1, B, slab_stride, topk, pad_value,
+                                            (hipStream_t)stream),
+                    "top-k row select launch");
 }
 
 size_t dsa_sparse_mla_workspace_bytes(int B, int H, int nsplit) {

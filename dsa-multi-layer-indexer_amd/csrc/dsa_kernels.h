@@ -98,6 +98,11 @@ hipError_t launch_topk_select(const float* scores, const int* seq_lens, const in
                               int pt_stride, void* scratch, int* out, int B, int slab, int K,
                               int sorted, int pad, hipStream_t s);
 
+// Sorted top-k, one workgroup a row (select_rows.hip): out int32 or int64.
+bool select_rows_takes(int B, int slab, int K);
+hipError_t launch_select_rows(const float* scores, const int* lens, void* out, int out64, int B, int slab, int K,
+                              int pad, hipStream_t s);
+
 // Prefill attention over bf16 keys (prefill.hip).  dtype: 0 fp32, 1 bf16, 2
 // fp16; mask == nullptr: causal only.
 size_t prefill_keys_bytes(int B, int T);

@@ -75,6 +75,8 @@ SIGNATURES = {
     "dsa_indexer_scan": (_i32, [_vp, _vp, _vp, _i64, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _vp]),
     "dsa_topk_scratch_bytes": (ctypes.c_size_t, [_i32, _i32]),
     "dsa_topk": (_i32, [_vp, _vp, _vp, _i32, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
+    "dsa_select_rows_supported": (_i32, [_i32, _i32, _i32]),
+    "dsa_select_rows": (_i32, [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _vp]),
     "dsa_sparse_mla_workspace_bytes": (ctypes.c_size_t, [_i32, _i32, _i32]),
     "dsa_sparse_mla_decode": (_i32, [_vp, _vp, _i64, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _vp]),
     "dsa_dense_mla_decode": (_i32, [_vp, _vp, _i64, _vp, _i32, _vp, _vp, _vp, _i32, _i32, _i32, _f32, _vp]),

@@ -112,6 +112,9 @@ def select_topk(logits: torch.Tensor, topk: int) -> torch.Tensor:
     if Skv > TOPK_MAX_CTX:
         raise ValueError(f"S_kv {Skv} above the select's limit {TOPK_MAX_CTX}")
     rows = logits.reshape(B * S, Skv).float().contiguous()
+    idx = ops.select_rows(rows, topk, pad_index(Skv))
+    if idx is not None:
+        return idx.reshape(B, S, topk)
     seq = torch.full((B * S,), Skv, dtype=torch.int32, device=logits.device)
     idx = ops.topk(rows, seq, topk, sorted=True, pad_value=pad_index(Skv))
     return idx.to(torch.int64).reshape(B, S, topk)

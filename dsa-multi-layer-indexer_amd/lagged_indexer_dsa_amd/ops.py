@@ -128,6 +128,18 @@ def topk(scores: torch.Tensor, seq_lens: torch.Tensor, k: int, sorted: bool = Fa
     return out
 
 
+def select_rows(scores: torch.Tensor, k: int, pad_value: int) -> torch.Tensor | None:
+    """:func:`topk` with sorted=True over whole rows, as int64 and in one
+    launch; None for the shapes the row kernel does not take."""
+    _dev(scores)
+    B, slab = scores.shape
+    if not _lib.load().dsa_select_rows_supported(B, slab, k):
+        return None
+    out = torch.empty(B, k, dtype=torch.int64, device=scores.device)
+    _lib.call("dsa_select_rows", scores.data_ptr(), None, out.data_ptr(), B, slab, k, pad_value, _stream())
+    return out
+
+
 def sparse_mla_workspace(B: int, H: int, nsplit: int, device) -> torch.Tensor:
     """Zero-filled workspace (split partials + the splits' barriers; every
     call leaves the barriers ready).  nsplit=0 sizes it for any split count."""

@@ -150,8 +150,9 @@ int dsa_indexer_scan(const void* q_fp8, const float* w, const void* index_k,
  *           scratch buffer.
  * DSA_TOPK_POSITION_ORDER runs as ONE launch: the workgroups of a row each
  * load a slice of its scores and select together (the decode layer's
- * cooperative select); DSA_TOPK_SORTED runs as two launches (histogram,
- * then per-slice filter and a sorting finalize).
+ * cooperative select); DSA_TOPK_SORTED runs as one launch of a workgroup a
+ * row (the scratch is not used), fewer than 24 rows of more than 131072 as
+ * two (histogram, then per-slice filter and a sorting finalize).
  * Requires topk <= 8192 (<= 4096 with DSA_TOPK_SORTED) and
  * slab_stride <= DSA_TOPK_MAX_CTX.
  * Replaces: reference attention_core.py:66-91 (select_topk), and on the GPU
@@ -163,6 +164,16 @@ int dsa_topk(const float* scores, const int32_t* seq_lens,
              const int32_t* page_table, int pt_stride, void* scratch,
              int32_t* out_idx, int B, int slab_stride, int topk, int flags,
              int32_t pad_value, void* stream);
+
+/*
+ * (2a) The sorted select of many rows with int64 indices and no scratch:
+ * DSA_TOPK_SORTED's order, pads and limits, for the shapes for which
+ * dsa_select_rows_supported returns 1.  seq_lens may be NULL (every row
+ * slab_stride long).
+ */
+int dsa_select_rows_supported(int B, int slab_stride, int topk);
+int dsa_select_rows(const float* scores, const int32_t* seq_lens, int64_t* out_idx, int B, int slab_stride, int topk,
+                    int32_t pad_value, void* stream);
 
 /*
  * (3) Split-K sparse MLA decode over the fp8 latent pool.
