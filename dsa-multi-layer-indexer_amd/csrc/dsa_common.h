@@ -31,6 +31,7 @@ struct PerDeviceOnce {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef uint32_t v2u_t __attribute__((ext_vector_type(2)));
 
 constexpr int kWave = 64;
 

@@ -15,12 +15,12 @@
 
 #include "dsa_common.h"
 #include "dsa_kernels.h"
+#include "quant_core.h"
 
 namespace dsa {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef uint32_t v2u __attribute__((ext_vector_type(2)));
 
 constexpr int kPfWaves = 4;                 // one per SIMD: the accumulators take half its registers
 constexpr int kPfThreads = kPfWaves * kWave;
@@ -311,10 +311,10 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_attention_kernel(const 
     for (int dt = 0; dt < 16; ++dt)
 #pragma unroll
       for (int i = 0; i < 16; i += 4) {
-        v2u w;
+        v2u_t w;
         w[0] = pack_bf16x2(o[dt][i] * inv, o[dt][i + 1] * inv);
         w[1] = pack_bf16x2(o[dt][i + 2] * inv, o[dt][i + 3] * inv);
-        *reinterpret_cast<v2u*>(orow + 32 * dt + 2 * i) = w;
+        *reinterpret_cast<v2u_t*>(orow + 32 * dt + 2 * i) = w;
       }
   } else {
     const long pr = ((long)sp * A.B + b) * R + row;
@@ -382,10 +382,10 @@ __global__ __launch_bounds__(kPfThreads) void prefill_merge_kernel(const Prefill
   if (threadIdx.x < 2 * kWave) {
     const int i = threadIdx.x;
     const v4f o = (so[0][i] + so[1][i]) + (so[2][i] + so[3][i]);
-    v2u w;
+    v2u_t w;
     w[0] = pack_bf16x2(o[0] * inv, o[1] * inv);
     w[1] = pack_bf16x2(o[2] * inv, o[3] * inv);
-    *reinterpret_cast<v2u*>(A.out + row * DSA_LATENT_DIM + 4 * i) = w;
+    *reinterpret_cast<v2u_t*>(A.out + row * DSA_LATENT_DIM + 4 * i) = w;
   }
 }
 
@@ -397,29 +397,6 @@ __global__ __launch_bounds__(kPfThreads) void prefill_merge_kernel(const Prefill
 // they hold (bf16_rn(e4m3 * scale), rope), 576 a row.  `stride` output rows a
 // request, those past T zero.  One wave a row: lane l holds dims 8l .. 8l + 7,
 // a group is 16 lanes, and lanes 0-7 take the rope.
-template <int DT>  // 0 fp32, 1 bf16, 2 fp16
-__device__ __forceinline__ void load8(const void* p, long i, float* x) {
-  if constexpr (DT == 0) {
-    const v4f* f = reinterpret_cast<const v4f*>(static_cast<const float*>(p) + i);
-    const v4f a = f[0], b = f[1];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] = a[e], x[4 + e] = b[e];
-  } else {
-    const uint4 v = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p) + i);
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if constexpr (DT == 1) {
-        x[2 * e] = bf16_lo(w[e]);
-        x[2 * e + 1] = bf16_hi(w[e]);
-      } else {
-        x[2 * e] = (float)__builtin_bit_cast(_Float16, (uint16_t)w[e]);
-        x[2 * e + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[e] >> 16));
-      }
-    }
-  }
-}
-
 template <int DT, bool ROWS>
 __global__ __launch_bounds__(kPfThreads) void pack_keys_kernel(const void* kv, uint8_t* out, int B, int T, int stride) {
   const long row = (long)blockIdx.x * kPfWaves + wave_id();
@@ -436,42 +413,24 @@ __global__ __launch_bounds__(kPfThreads) void pack_keys_kernel(const void* kv, u
   float x[8], r[8];
   load8<DT>(kv, src + 8 * lane, x);
   if (lane < 8) load8<DT>(kv, src + DSA_LATENT_DIM + 8 * lane, r);
-  // |x| as integer bits: NaN above infinity above every finite value
-  uint32_t am = 0;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) am = max(am, __float_as_uint(x[e]) & 0x7fffffffu);
-#pragma unroll
-  for (int d = 1; d < 16; d <<= 1) am = max(am, (uint32_t)__shfl_xor((int)am, d));
-  const float amax = __uint_as_float(am);
-  const float scale = (amax < 1e-6f ? 1e-6f : amax) / 448.f;
-  int code[4];
-#pragma unroll
-  for (int e = 0; e < 8; e += 2) {
-    float y0 = x[e] / scale, y1 = x[e + 1] / scale;
-    // the comparisons are false for NaN, which stays
-    y0 = y0 > 448.f ? 448.f : (y0 < -448.f ? -448.f : y0);
-    y1 = y1 > 448.f ? 448.f : (y1 < -448.f ? -448.f : y1);
-    code[e >> 1] = __builtin_amdgcn_cvt_pk_fp8_f32(y0, y1, 0, false);
-  }
+  const float scale = row_scale<true>(x);
+  const v2u_t code = quant8<true>(x, scale);
   uint32_t rope[4] = {0, 0, 0, 0};
   if (lane < 8)
 #pragma unroll
     for (int e = 0; e < 4; ++e) rope[e] = pack_bf16x2(r[2 * e], r[2 * e + 1]);
   if constexpr (ROWS) {
-    v2u c;
-    c[0] = ((uint32_t)code[0] & 0xffffu) | (uint32_t)code[1] << 16;
-    c[1] = ((uint32_t)code[2] & 0xffffu) | (uint32_t)code[3] << 16;
-    *reinterpret_cast<v2u*>(dst + 8 * lane) = c;
+    *reinterpret_cast<v2u_t*>(dst + 8 * lane) = code;
     if ((lane & 15) == 0) *reinterpret_cast<float*>(dst + DSA_LATENT_DIM + (lane >> 2)) = scale;
     if (lane < 8)
       *reinterpret_cast<uint4*>(dst + DSA_LATENT_DIM + 16 + 16 * lane) = make_uint4(rope[0], rope[1], rope[2], rope[3]);
   } else {
+    float f[8];
+    e4m3x4_to_f32(code[0], f);
+    e4m3x4_to_f32(code[1], f + 4);
     uint32_t w[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const auto f = __builtin_amdgcn_cvt_pk_f32_fp8(code[e], false);
-      w[e] = pack_bf16x2(f[0] * scale, f[1] * scale);
-    }
+    for (int e = 0; e < 4; ++e) w[e] = pack_bf16x2(f[2 * e] * scale, f[2 * e + 1] * scale);
     // A tile holds keys that some of its rows do not attend, and 0 * NaN
     // would reach those rows' outputs: a key with a non-finite latent value
     // (its score is NaN whatever the query) keeps a NaN in its rope, which
