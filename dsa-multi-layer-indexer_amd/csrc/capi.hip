@@ -684,6 +684,27 @@ int dsa_prefill_attention(const void* q_bf16, const void* keys, const uint32_t* 
                     "prefill attention");
 }
 
+size_t dsa_prefill_logits_workspace_bytes(int B, int S, int H, int T) {
+  return B < 1 || S < 1 || H < 1 || T < 1 ? 0 : dsa::prefill_logits_workspace_bytes(B, S, H, T);
+}
+
+int dsa_prefill_logits(const void* q, int q_dtype, const void* k, int k_dtype, const void* w, int w_dtype,
+                       void* workspace, float* logits, int B, int S, int H, int T, void* stream) {
+  DSA_REQUIRE(q && k && w && workspace && logits, DSA_ERR_INVALID_ARG, "dsa_prefill_logits: null pointer");
+  DSA_REQUIRE(B >= 1 && S >= 1 && T >= 1 && T <= 1 << 28, DSA_ERR_INVALID_ARG, "dsa_prefill_logits: bad shape B=%d S=%d T=%d",
+              B, S, T);
+  DSA_REQUIRE((int64_t)B * S <= 65535, DSA_ERR_UNSUPPORTED, "dsa_prefill_logits: B * S must be <= 65535");
+  DSA_REQUIRE(H >= 16 && H <= 64 && H % 16 == 0, DSA_ERR_UNSUPPORTED,
+              "dsa_prefill_logits: index_n_heads must be 16, 32, 48 or 64 (got %d)", H);
+  DSA_REQUIRE(q_dtype >= 0 && q_dtype <= 2 && k_dtype >= 0 && k_dtype <= 2 && w_dtype >= 0 && w_dtype <= 2,
+              DSA_ERR_INVALID_ARG, "dsa_prefill_logits: dtypes must be 0 (fp32), 1 (bf16) or 2 (fp16)");
+  DSA_REQUIRE(aligned16(q) && aligned16(k) && aligned16(workspace), DSA_ERR_INVALID_ARG,
+              "dsa_prefill_logits: q, k and workspace must be 16-byte aligned");
+  return hip_status(dsa::launch_prefill_logits(q, q_dtype, k, k_dtype, w, w_dtype, workspace, logits, B, S, H, T,
+                                               (hipStream_t)stream),
+                    "prefill logits");
+}
+
 int dsa_append_latent_rows(const void* latent_bf16, const int32_t* slots, int n, void* kv_pool, int64_t kv_rows,
                            void* stream) {
   DSA_REQUIRE(n >= 0, DSA_ERR_INVALID_ARG, "dsa_append_latent_rows: n must be >= 0 (got %d)", n);

@@ -115,6 +115,12 @@ hipError_t launch_selection_set(const void* idx, int idx64, int rows, int n, int
 hipError_t launch_prefill_attention(const void* q, const void* keys, const uint32_t* mask, void* workspace, void* out,
                                     int B, int S, int H, int T, float sm_scale, hipStream_t s);
 
+// Indexer scores of many query rows (prefill_logits.hip); qt, kt, wt: the
+// inputs' element types as above.
+size_t prefill_logits_workspace_bytes(int B, int S, int H, int T);
+hipError_t launch_prefill_logits(const void* q, int qt, const void* k, int kt, const void* w, int wt, void* workspace,
+                                 float* out, int B, int S, int H, int T, hipStream_t s);
+
 // Decode-step operand preparation (quant.hip).
 hipError_t launch_quant_query(const void* q_bf16, const float* w, void* codes, float* w_out, long rows,
                               hipStream_t s);

@@ -91,6 +91,8 @@ SIGNATURES = {
     "dsa_quantize_index_query": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _vp]),
     "dsa_append_index_keys": (_i32, [_vp, _vp, _vp, _i32, _vp, _i32, _vp, _i64, _vp]),
     "dsa_append_latent_rows": (_i32, [_vp, _vp, _i32, _vp, _i64, _vp]),
+    "dsa_prefill_logits_workspace_bytes": (ctypes.c_size_t, [_i32, _i32, _i32, _i32]),
+    "dsa_prefill_logits": (_i32, [_vp, _i32, _vp, _i32, _vp, _i32, _vp, _vp, _i32, _i32, _i32, _i32, _vp]),
     "dsa_prefill_keys_bytes": (ctypes.c_size_t, [_i32, _i32]),
     "dsa_prefill_workspace_bytes": (ctypes.c_size_t, [_i32, _i32, _i32, _i32]),
     "dsa_selection_bits_bytes": (ctypes.c_size_t, [_i32, _i32]),

@@ -36,8 +36,8 @@ from __future__ import annotations
 
 import torch
 
-from . import formats, ops
-from ._lib import INDEX_DIM, LATENT_DIM, PAGE_TOKENS, QK_DIM, SELECTION_MAX_CTX, TOPK_MAX_CTX
+from . import ops
+from ._lib import INDEX_DIM, LATENT_DIM, QK_DIM, SELECTION_MAX_CTX, TOPK_MAX_CTX
 
 def _gpu(*ts: torch.Tensor) -> None:
     for t in ts:
@@ -71,25 +71,9 @@ def indexer_logits(index_q: torch.Tensor, index_k: torch.Tensor, weights: torch.
     if D != INDEX_DIM:
         raise ValueError(f"the fp8 indexer contracts D = {INDEX_DIM}, got {D}")
     _gpu(index_q, index_k, weights)
-    dev = index_q.device
-    Skv = index_k.shape[1]
-    npg = max(1, (Skv + PAGE_TOKENS - 1) // PAGE_TOKENS)
-    # identity paging: batch b's page p is physical page b * npg + p; every
-    # key of the batch quantized in one call and laid out page by page
-    pt = (torch.arange(B, dtype=torch.int32, device=dev)[:, None] * npg
-          + torch.arange(npg, dtype=torch.int32, device=dev)[None, :])
-    codes, sc = formats.quantize_rowwise(index_k.reshape(B * Skv, D))
-    kpad = torch.zeros(B, npg * PAGE_TOKENS, D, dtype=torch.uint8, device=dev)
-    kpad[:, :Skv] = codes.reshape(B, Skv, D)
-    spad = torch.zeros(B, npg * PAGE_TOKENS, dtype=torch.float32, device=dev)
-    spad[:, :Skv] = sc.reshape(B, Skv)
-    pages = torch.cat([kpad.reshape(B * npg, PAGE_TOKENS * D),
-                       spad.reshape(B * npg, PAGE_TOKENS).view(torch.uint8)], dim=1).contiguous()
-    q8, wq = formats.quantize_index_query(index_q.reshape(B * S, H, D), weights.reshape(B * S, H))
-    rows_pt = pt.repeat_interleave(S, dim=0).contiguous()
-    seq = torch.full((B * S,), Skv, dtype=torch.int32, device=dev)
-    scores = ops.indexer_scan(q8, wq, pages, rows_pt, seq, npg * PAGE_TOKENS)
-    return scores[:, :Skv].reshape(B, S, Skv)
+    if index_k.shape[1] == 0:  # no key
+        return torch.empty(B, S, 0, dtype=torch.float32, device=index_q.device)
+    return ops.prefill_logits(index_q, index_k, weights)
 
 
 def apply_causal_mask(logits: torch.Tensor) -> torch.Tensor:

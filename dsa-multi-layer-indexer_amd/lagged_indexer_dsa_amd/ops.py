@@ -243,15 +243,34 @@ def dense_mla_decode(q: torch.Tensor, kv_pool: torch.Tensor, page_table: torch.T
 _PACK_DTYPES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 
 
+def _kernel_input(x: torch.Tensor) -> torch.Tensor:
+    """x as the prefill kernels read it: fp32, bf16 or fp16, contiguous,
+    16-byte aligned."""
+    x = (x if x.dtype in _PACK_DTYPES else x.float()).contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
 def _pack_source(kv: torch.Tensor) -> torch.Tensor:
-    """kv [B, T, 576] as the pack kernels read it: fp32, bf16 or fp16,
-    contiguous, 16-byte aligned."""
+    """kv [B, T, 576] as the pack kernels read it (rope rounded to bf16 once)."""
     if kv.dtype not in _PACK_DTYPES:
         x = kv.float()
         x[..., LATENT_DIM:] = kv[..., LATENT_DIM:].to(torch.bfloat16)
         kv = x
-    kv = kv.contiguous()
-    return kv if kv.data_ptr() % 16 == 0 else kv.clone()
+    return _kernel_input(kv)
+
+
+def prefill_logits(q: torch.Tensor, k: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """Indexer scores [B, S, T] fp32 of q [B, S, H, 128] and w [B, S, H] over
+    k [B, T, 128], quantised per row inside.  Reference: attention_core.py:27-49."""
+    q, k, w = _kernel_input(q), _kernel_input(k), _kernel_input(w)
+    _dev(q, k, w)
+    B, S, H, _ = q.shape
+    T = k.shape[1]
+    ws = torch.empty(_lib.load().dsa_prefill_logits_workspace_bytes(B, S, H, T), dtype=torch.uint8, device=q.device)
+    out = torch.empty(B, S, T, dtype=torch.float32, device=q.device)
+    _lib.call("dsa_prefill_logits", q.data_ptr(), _PACK_DTYPES[q.dtype], k.data_ptr(), _PACK_DTYPES[k.dtype],
+              w.data_ptr(), _PACK_DTYPES[w.dtype], ws.data_ptr(), out.data_ptr(), B, S, H, T, _stream())
+    return out
 
 
 def pack_latent_rows(kv: torch.Tensor, row_stride: int) -> torch.Tensor:

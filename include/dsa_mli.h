@@ -368,6 +368,21 @@ int dsa_append_latent_rows(const void* latent_bf16, const int32_t* slots, int n,
                            void* stream);
 
 /*
+ * (6a) Indexer scores of S query rows per request against its T keys, no
+ * causal masking: logits[b, s, g] = s_k[g] * sum_h w'[b, s, h] *
+ * ReLU(q8[b, s, h] . k8[b, g]), q and k quantised by (6)'s rule inside (a NaN
+ * in a row makes its scale NaN), w' = w * s_q.
+ *   q [B, S, H, 128], k [B, T, 128], w [B, S, H] (dtype 0 fp32, 1 bf16, 2
+ *   fp16, each its own); logits [B, S, T] fp32; workspace
+ *   dsa_prefill_logits_workspace_bytes(B, S, H, T) bytes (no
+ *   initialisation); H 16, 32, 48 or 64; B * S <= 65535.
+ * Replaces: indexer_logits (attention_core.py:27-49) over many query rows.
+ */
+size_t dsa_prefill_logits_workspace_bytes(int B, int S, int H, int T);
+int dsa_prefill_logits(const void* q, int q_dtype, const void* k, int k_dtype, const void* w, int w_dtype,
+                       void* workspace, float* logits, int B, int S, int H, int T, void* stream);
+
+/*
  * (7) Prefill attention: S query rows at the end of each request's T keys.
  * Row s of request b sees keys 0 .. T - S + s; all heads share the keys.
  *
