@@ -1096,7 +1096,8 @@ __device__ __forceinline__ void coop_select(CoopShared& cs, unsigned char* smem,
   } else {
     // t* must be >= L = the largest list bound for the lists to hold every
     // key >= t*; keys below L never matter.
-    const uint32_t lo = max(h0, kKeyNegInf), hi = h1;
+    uint32_t lo = max(h0, kKeyNegInf);
+    const uint32_t hi = h1;
     bool ok = hi >= lo;
     uint32_t T1 = 0, above = 0, nbin = 0;
     int sh = 0;
@@ -1121,6 +1122,30 @@ __device__ __forceinline__ void coop_select(CoopShared& cs, unsigned char* smem,
       T1 = th.bin;                   // == (t* - lo) >> sh
       above = th.above;
       nbin = th.cnt;
+      // A bin of more than one wave's keys is split again, 2048 ways.  Short
+      // rows need it: their lists hold every key, so the window runs from the
+      // most negative score, its bins are a quarter of an exponent wide and the
+      // threshold's holds hundreds of keys, each of which rank counting below
+      // compared with every other (a layer of 4133 tokens 19.2 us, split
+      // 14.8; four such rows 27.3, 17.5; 131072 tokens, where the first
+      // window is enough, 14.9 and 14.8).
+      while (ok && nbin > (uint32_t)kWave && sh > 0) {  // uniform
+        const int width = sh;
+        lo += T1 << sh;
+        sh = max(0, sh - 11);
+        __syncthreads();
+        for (int i = t; i < kUnionWords / 4; i += kMainThreads)
+          reinterpret_cast<uint4*>(hist)[i] = make_uint4(0, 0, 0, 0);
+        __syncthreads();
+        for_mine([&](uint32_t w, uint32_t) {  // (a key below lo wraps past the bin)
+          if ((w - lo) >> width == 0u) atomicAdd(&hist[union_slot((w - lo) >> sh)], 1u);
+        });
+        __syncthreads();
+        const BinThreshold ts = wave_threshold_sum<kUnionGroup, kUnionStride>(hist, (uint32_t)K - above);
+        T1 = ts.bin;
+        above += ts.above;
+        nbin = ts.cnt;
+      }
     }
     dbg_stamp(dbk, 4);
     if (!ok) {
@@ -2044,7 +2069,7 @@ void attn_bind_workspace(AttnArgs& A, void* ws, int B) {
 static int g_scan_blocks_cap = 0;  // internal: cap on scan workgroups per launch (0 = none)
 void set_scan_blocks_cap(int n) { g_scan_blocks_cap = std::max(0, n); }
 
-int scan_blocks_per_row(int B, int pt_stride, int slab_stride, int att_blocks, bool big_lds) {
+int scan_blocks_per_row(int B, int pt_stride, int slab_stride, int att_blocks, bool big_lds, bool select) {
   const long cap = std::min((long)slab_stride, (long)pt_stride * DSA_PAGE_TOKENS);
   const long cap_chunks = (cap + kChunkKeys - 1) / kChunkKeys;
   const int cus = device_cus();
@@ -2053,7 +2078,12 @@ int scan_blocks_per_row(int B, int pt_stride, int slab_stride, int att_blocks, b
   long target = big_lds ? std::max<long>(cus - att_blocks, cus / 2) : 2L * cus;
   if (g_scan_blocks_cap > 0) target = std::min<long>(target, g_scan_blocks_cap);
   long per_row = (target + B - 1) / B;
-  per_row = std::min(per_row, std::max(1L, cap_chunks / kMainWaves));
+  // short rows: a chunk a wave in a plain scan; at least 4 chunks a workgroup
+  // when it also selects, which leaves waves without keys but shortens the
+  // lists, the steps that pace the select (a layer of 4133 tokens 14.8 us with
+  // 32 workgroups, 12.9 with 64; 2 chunks the same, 1 chunk, 224 workgroups,
+  // 21.8; 8192 tokens 14.1 and 12.5; from 16384 tokens the target decides)
+  per_row = std::min(per_row, std::max(1L, cap_chunks / (select ? 4 : kMainWaves)));
   // each workgroup's page-table entries must fit the LDS table
   const long cap_pages = (cap + DSA_PAGE_TOKENS - 1) / DSA_PAGE_TOKENS;
   per_row = std::max(per_row, (cap_pages + kScanMaxPages - 3) / (kScanMaxPages - 2));
@@ -2132,7 +2162,7 @@ hipError_t launch_decode_main(const AttnArgs* A, int B_att, const ScanArgs* S, i
   if (S) {
     sc = *S;
     sc.blocks_per_row = scan_blocks_per_row(B_scan, sc.pt_stride, sc.slab_stride, n_att,
-                                            n_att > 0 || select);
+                                            n_att > 0 || select, select);
     sc.coop = 0;
     if (select && g_coop_select) {
       // cooperative select: the row's workgroups wait for each other, so
