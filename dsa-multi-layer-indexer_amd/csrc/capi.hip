@@ -183,6 +183,11 @@ dsa::ScanArgs scan_args(const void* q_fp8, const float* w, const void* index_k, 
   return S;
 }
 
+// The attention by itself: entries (3), (3a) and (3b).
+hipError_t launch_attention(const dsa::AttnArgs& A, int B, hipStream_t s) {
+  return dsa::mla_rows_takes(A, B) ? dsa::launch_mla_rows(A, B, s) : dsa::launch_decode_main(&A, B, nullptr, 0, s);
+}
+
 // Rows from which a layer's indexer runs as two launches (scan, then select
 // beside the attention) instead of one: the fused launch pins one workgroup
 // per CU for the whole scan, which large batches cannot afford.
@@ -472,7 +477,7 @@ int dsa_sparse_mla_decode(const void* q_bf16, const void* kv_pool, int64_t kv_ro
   if (rc) return rc;
   dsa::AttnArgs A = attn_args(q_bf16, kv_pool, kv_rows, idx, workspace, out_bf16, B, H, topk,
                               nsplit, sm_scale);
-  return hip_status(dsa::launch_decode_main(&A, B, nullptr, 0, (hipStream_t)stream),
+  return hip_status(launch_attention(A, B, (hipStream_t)stream),
                     "sparse MLA launch");
 }
 
@@ -489,7 +494,7 @@ int dsa_dense_mla_decode(const void* q_bf16, const void* kv_pool, int64_t kv_row
   if (rc) return rc;
   dsa::AttnArgs A = dense_attn_args(q_bf16, kv_pool, kv_rows, page_table, pt_stride, seq_lens, workspace,
                                     out_bf16, B, H, nsplit, sm_scale);
-  return hip_status(dsa::launch_decode_main(&A, B, nullptr, 0, (hipStream_t)stream), "dense MLA launch");
+  return hip_status(launch_attention(A, B, (hipStream_t)stream), "dense MLA launch");
 }
 
 int dsa_sparse_mla_decode_noalloc(const void* q_bf16, const void* kv_pool, int64_t kv_rows,
@@ -514,7 +519,7 @@ int dsa_sparse_mla_decode_noalloc(const void* q_bf16, const void* kv_pool, int64
   A.sync = reinterpret_cast<uint32_t*>(base);
   A.part_o = reinterpret_cast<float*>(static_cast<unsigned char*>(base) + kNoAllocSyncBytes);
   A.part_ml = A.part_o + (size_t)groups * ns * 16 * DSA_LATENT_DIM;
-  return hip_status(dsa::launch_decode_main(&A, B, nullptr, 0, (hipStream_t)stream),
+  return hip_status(launch_attention(A, B, (hipStream_t)stream),
                     "sparse MLA (no-alloc) launch");
 }
 

@@ -77,24 +77,6 @@ __device__ __forceinline__ v4f mfma_bf16(const uint4& a, const uint4& b, v4f c) 
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, c, 0, 0, 0);
 }
 
-// 16 e4m3 (one uint4) * scale -> 16 bf16 (two uint4: elements 0-7, 8-15),
-// bf16_rn(f32(e4m3) * scale) exactly.
-__device__ __forceinline__ void dequant16(const uint4& v, float sc, uint4& lo, uint4& hi) {
-  float f[16];
-  e4m3x4_to_f32(v.x, f + 0);
-  e4m3x4_to_f32(v.y, f + 4);
-  e4m3x4_to_f32(v.z, f + 8);
-  e4m3x4_to_f32(v.w, f + 12);
-  lo.x = pack_bf16x2(f[0] * sc, f[1] * sc);
-  lo.y = pack_bf16x2(f[2] * sc, f[3] * sc);
-  lo.z = pack_bf16x2(f[4] * sc, f[5] * sc);
-  lo.w = pack_bf16x2(f[6] * sc, f[7] * sc);
-  hi.x = pack_bf16x2(f[8] * sc, f[9] * sc);
-  hi.y = pack_bf16x2(f[10] * sc, f[11] * sc);
-  hi.z = pack_bf16x2(f[12] * sc, f[13] * sc);
-  hi.w = pack_bf16x2(f[14] * sc, f[15] * sc);
-}
-
 typedef short v4s __attribute__((ext_vector_type(4)));
 
 // B operand of the PV MFMA (k = 32 keys, n = 16 dims) from the row-major

@@ -88,6 +88,11 @@ int attn_fused_nsplit(int topk, int B, int H);
 size_t attn_workspace_bytes(int B, int H, int nsplit);
 void attn_bind_workspace(AttnArgs& A, void* ws, int B);
 
+// The same attention for workgroups of many keys (mla_rows.hip): whether it
+// takes A (its split count resolved), and its launch.
+bool mla_rows_takes(const AttnArgs& A, int B);
+hipError_t launch_mla_rows(const AttnArgs& A, int B, hipStream_t s);
+
 // Top-k: histogram (standalone) + select (filter, last arriver finalizes).
 size_t topk_scratch_bytes(int B, int slab);
 size_t row_select_lds_bytes();

@@ -21,7 +21,8 @@ CSRC = ROOT_DIR / "csrc"
 INCLUDE = REPO_DIR / "include"
 LIB_DIR = PKG_DIR / "_lib"
 LIB_PATH = LIB_DIR / "libdsa_mli.so"
-SOURCES = ["libdsa_mli.hip", "capi.hip", "prefill.hip", "prefill_logits.hip", "select_rows.hip", "quant.hip", "sol.hip"]
+SOURCES = ["libdsa_mli.hip", "capi.hip", "mla_rows.hip", "prefill.hip", "prefill_logits.hip", "select_rows.hip",
+           "quant.hip", "sol.hip"]
 ARCH = "gfx950"
 
 

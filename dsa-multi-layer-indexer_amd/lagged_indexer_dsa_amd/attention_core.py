@@ -115,11 +115,12 @@ def _attend_by_tiles(B: int, S: int, H: int, Skv: int, n: int) -> bool:
     others, or gathered row by row.
 
     With the chip full (4096 rows and more) a gathered key costs about what
-    3.5 to 4 streamed ones do (1024 queries x 16 heads, top-2048: 4096 tokens
-    180 us against 289, 8192 tokens 312 against 298, 16384 tokens 570 against
-    310); with fewer rows the gather spreads over the idle CUs and the line
+    2.5 streamed ones do (1024 queries x 16 heads, top-2048: 4096 tokens
+    189 us against 236, 5120 tokens 224 against 236, 6144 tokens 261 against
+    234, 8192 tokens 325 against 230; 2048 queries, 6144 tokens 411 against
+    424); with fewer rows the gather spreads over the idle CUs and the line
     lies near 2 (100 queries, top-2048: 2048 tokens 45 against 52, 4096 equal,
-    8192 69 against 57); with a handful of queries both are a few launches
+    8192 69 against 57; 200 queries, 4096 equal); with a handful of queries both are a few launches
     and splitting the stream over the CUs is as quick up to a few thousand
     tokens (4 queries: 4096 tokens 33 against 43 us, 12000 tokens 44 against
     43; 16 queries: 2048 tokens 37 against 43, 4096 tokens 45 against 43)."""
@@ -129,7 +130,7 @@ def _attend_by_tiles(B: int, S: int, H: int, Skv: int, n: int) -> bool:
         return visible <= 8192
     if rows <= 256:
         return visible <= 4096
-    return visible <= (3.5 if rows >= 4096 else 2.0) * n
+    return visible <= (2.5 if rows >= 4096 else 2.0) * n
 
 
 def _attend_rows(q: torch.Tensor, kv: torch.Tensor, idx: torch.Tensor, sm_scale: float) -> torch.Tensor:
