@@ -102,10 +102,14 @@ __device__ __forceinline__ uint4 load_v_operand(const uint16_t* vt, int key0, in
 // (attention-only launches); otherwise each key wave loads its operand from
 // memory (the fused launch: measured 0.13 us per C3 layer faster that way,
 // while an attention-only launch is 0.3 us faster staged).
-template <bool STAGE_Q>
-__device__ __forceinline__ void attention_block(const AttnArgs& A, int b, int hg, int sp, unsigned char* smem) {
+// BY_LEN (dense rows): the row's own number of splits, which divide its
+// length (dense_rows_kernel), its partials from part0 on; otherwise A.nsplit
+// splits of every row, which divide what a row may hold.
+template <bool STAGE_Q, bool BY_LEN = false>
+__device__ __forceinline__ void attention_block(const AttnArgs& A, int b, int hg, int sp, unsigned char* smem,
+                                                int row_splits = 0, long part0 = 0) {
   AttnShared& sh = *reinterpret_cast<AttnShared*>(smem);
-  const int nhg = A.H / kHG, nsplit = A.nsplit;
+  const int nhg = A.H / kHG, nsplit = BY_LEN ? row_splits : A.nsplit;
   const int dbk = blockIdx.x;
   dbg_stamp(dbk, 0);
   const int t = threadIdx.x;
@@ -115,8 +119,9 @@ __device__ __forceinline__ void attention_block(const AttnArgs& A, int b, int hg
   // the barrier's flag value, read now and used at the barrier (the load's
   // latency hides under the gather)
   const uint32_t sense = (t == 0) ? group_sense(A.sync + ((long)b * nhg + hg) * kSyncWords, sp) : 0u;
-  const int kps = (A.topk + nsplit - 1) / nsplit;
-  const int k0 = min(A.topk, sp * kps), k1 = min(A.topk, k0 + kps);
+  const int keys = BY_LEN ? max(0, min(A.dense_lens[b], A.topk)) : A.topk;
+  const int kps = (keys + nsplit - 1) / nsplit;
+  const int k0 = min(keys, sp * kps), k1 = min(keys, k0 + kps);
   // the KV slot of key j of the row: the selection's entry, or (dense) the
   // slot of token j through the page table (-1 at or past the row's length)
   const int* idx_row = A.idx + (long)b * A.topk;
@@ -324,7 +329,7 @@ __device__ __forceinline__ void attention_block(const AttnArgs& A, int b, int hg
   // 64wv + 16nt + kr, one 16-byte store, so each wave store writes 1 KB
   // contiguous (16 dims x 16 heads; per-element stores of a [head][dim]
   // layout took ~0.8 us to issue).  (m, l) per head, log2 domain.
-  const long pblk0 = ((long)b * nhg + hg) * nsplit;
+  const long pblk0 = BY_LEN ? part0 : ((long)b * nhg + hg) * nsplit;
   const long pblk = pblk0 + sp;
   {
     const __amdgpu_buffer_rsrc_t pw = dev_rsrc(A.part_o + pblk * (kHG * DSA_LATENT_DIM), kHG * DSA_LATENT_DIM * 4u);
@@ -1925,6 +1930,39 @@ __global__ __launch_bounds__(kMainThreads, (ROLES & ~kRolePlan) == kRoleScan ? 4
   }
 }
 
+// Dense rows by themselves, the launch's workgroups divided over them by
+// length: of a head group's W = B * A.nsplit workgroups every row gets one,
+// and of the rest its share of all keys (at most one for 64 keys, and
+// kMaxSplit; the products stay below 2^32: W < 256, u <= 2^24).  A.nsplit
+// splits of every row's capacity leave the workgroups of short rows idle:
+// rows of 777, 20000 and 32768 keys x 64 heads took 59.5 us, the longest
+// one's splits holding 1561 keys; now 850, and 44.4.  Eight rows of 500 to
+// 16000 keys x 64 heads: 69.5 -> 39.3; 30 rows of 2000 keys in a table of
+// the same size 48 -> 42.5 (spare workgroups used); rows of equal length
+// that fill their tables keep their splits and pay for the lengths being
+// read first: 4 x 5000 keys 15.2 -> 15.5, 2 x 131072 keys 50.4 -> 50.9.
+// What bounds it now is the 128-key tile, ~4 us, times the tiles a split
+// holds.  A head group's workgroups are contiguous in the grid, as the other
+// launches' splits of a (row, head group) are.
+__global__ __launch_bounds__(kMainThreads, 1) void dense_rows_kernel(AttnArgs A, int B) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  dbg_begin();
+  const int W = B * A.nsplit, hg = blockIdx.x / W, w = blockIdx.x % W;
+  const int lane = threadIdx.x & (kWave - 1);
+  const bool in = lane < B;
+  const uint32_t u = in ? ((uint32_t)max(0, min(A.dense_lens[lane], A.topk)) + 63u) / 64u : 0u;
+  const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_incl<0>(u), kWave - 1);
+  uint32_t n = 0;
+  if (in) n = all ? min(min(1u + (uint32_t)(W - B) * u / all, (uint32_t)kMaxSplit), max(u, 1u)) : 1u;
+  const uint32_t incl = wave_scan_incl<0>(n);
+  const uint64_t m = __ballot(in && incl > (uint32_t)w);
+  if (!m) return;  // a spare workgroup
+  const int b = __builtin_ctzll(m);
+  const int nrow = __builtin_amdgcn_readlane((int)n, b), first = __builtin_amdgcn_readlane((int)(incl - n), b);
+  attention_block<true, true>(A, b, hg, w - first, smem, nrow, (long)hg * W + first);
+  dbg_flush(blockIdx.x);
+}
+
 // ---------------------------------------------------------------- host side
 static int g_scan_variant = 0;
 void set_scan_variant(int v) { g_scan_variant = v ? 1 : 0; }
@@ -2123,6 +2161,13 @@ static int g_flat_scan = 1;  // internal switch: plain scans of >= 2 rows throug
 void set_flat_scan(int on) { g_flat_scan = on ? 1 : 0; }
 bool flat_scan_on() { return g_flat_scan != 0; }
 
+// Splits of dense rows by length: from two rows on (one has nothing to share
+// out), as many as a wave has lanes, when all workgroups are resident (a
+// row's may be anywhere in its head group's).
+static bool dense_by_len(const AttnArgs& a, int B, int blocks) {
+  return a.dense_pt && a.nsplit > 1 && B >= 2 && B <= kWave && blocks <= device_cus();
+}
+
 hipError_t launch_decode_main(const AttnArgs* A, int B_att, const ScanArgs* S, int B_scan,
                               hipStream_t s) {
 #ifndef DSA_FLAT_MIN_ROWS
@@ -2181,6 +2226,15 @@ hipError_t launch_decode_main(const AttnArgs* A, int B_att, const ScanArgs* S, i
     sc.target = big_lds ? std::max(device_cus() - n_att, device_cus() / 2) : n_scan;
   }
   if (n_att + n_scan == 0) return hipSuccess;
+  if (A && !S && dense_by_len(a, B_att, n_att)) {
+    static PerDeviceOnce attr;
+    const hipError_t e = attr.run([&] {
+      return hipFuncSetAttribute((const void*)dense_rows_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_attn);
+    });
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(dense_rows_kernel, dim3(n_att), dim3(kMainThreads), lds_attn, s, a, B_att);
+    return hipGetLastError();
+  }
   size_t lds = sizeof(ScanShared);
   if (n_att) lds = std::max(lds, lds_attn);
   if (select) lds = std::max(lds, sc.coop ? lds_coop : (size_t)kRowSelWords * 4);
