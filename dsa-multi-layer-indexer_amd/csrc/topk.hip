@@ -7,6 +7,10 @@
 // the radix-select structure of the GPU selectors (tilelang_dsa/
 // topk_selector.py:36-194; in-kernel exact select K:1097-1129, K:1248-1310).
 //
+// The sorted select of many rows, or of rows up to 131072 scores, is
+// select_rows.hip's; this file's form is for a few longer rows and top-k
+// above its limit.
+//
 // Two launches (the histogram is fused into the indexer scan on the decode
 // path, leaving one), so a 128K-196K row is read by many CUs:
 //   (A) histogram: workgroups over 4096-score slices build an LDS histogram
