@@ -206,7 +206,8 @@ int dsa_sparse_mla_decode(const void* q_bf16, const void* kv_pool,
  * keys 0..seq_lens[b]-1 at KV slots page_table[b*pt_stride + j/64]*64 + j%64
  * (seq_lens clamped to pt_stride*64).  workspace:
  * dsa_sparse_mla_workspace_bytes(B, H, nsplit), as for (3); nsplit = 0:
- * one split per 64 keys of the page table's capacity, at most 128.
+ * one split per 64 keys of the page table's capacity, at most 128.  From 2 to
+ * 64 rows whose splits are all resident share B * nsplit splits by length.
  * Replaces: dense_mla_core (attention_core.py:142-160), the full-attention
  * layers and the DENSE cold start of DSAModel.forward (model.py:51-59,
  * 104-114).
