@@ -1124,8 +1124,10 @@ __device__ __forceinline__ void coop_select(CoopShared& cs, unsigned char* smem,
         for (int i = t; i < kUnionWords / 4; i += kMainThreads)
           reinterpret_cast<uint4*>(hist)[i] = make_uint4(0, 0, 0, 0);
         __syncthreads();
-        for_mine([&](uint32_t w, uint32_t) {  // (a key below lo wraps past the bin)
-          if ((w - lo) >> width == 0u) atomicAdd(&hist[union_slot((w - lo) >> sh)], 1u);
+        // (w >= lo: NaN's bin begins within a bin's width of 2^32, where w - lo
+        // of the lists' zero padding would wrap into it)
+        for_mine([&](uint32_t w, uint32_t) {
+          if (w >= lo && (w - lo) >> width == 0u) atomicAdd(&hist[union_slot((w - lo) >> sh)], 1u);
         });
         __syncthreads();
         const BinThreshold ts = wave_threshold_sum<kUnionGroup, kUnionStride>(hist, (uint32_t)K - above);

@@ -71,3 +71,51 @@ def test_short_layers(dev, lens):
         ref = O.topk_select(L.scores.cpu().numpy(), np.array(lens), L.topk, page_table=pt.cpu().numpy())
         assert np.array_equal(L.next_idx.cpu().numpy(), ref)
     assert _lib.sync_timeouts() == 0
+
+
+# Rows whose K-th key is NaN (ranked above +inf): nothing finite is selected,
+# the row is all pads.  The threshold bin is then the topmost one, next to
+# 2^32, and the lists' zero padding must not count in it.
+@pytest.mark.parametrize("nans", ["many", "k", "k-1"])
+@pytest.mark.parametrize("lens,k", [([2600], 2048), ([3000], 2048), ([4133], 2048), ([8192], 512), ([1030], 1024),
+                                    ([20000], 2048), ([131072], 2048), ([4133, 2100, 70, 6000], 2048)])
+def test_rows_of_nans(dev, lens, k, nans):
+    from lagged_indexer_dsa_amd import _lib, ops
+
+    _lib.sync_timeouts(reset=True)
+    rng = np.random.default_rng(k + sum(lens))
+    x = rng.standard_normal((len(lens), max(lens))).astype(np.float32)
+    for r, n in enumerate(lens):
+        count = {"many": k + (n - k) // 3, "k": k, "k-1": k - 1}[nans] if n > k else n // 2
+        x[r, rng.permutation(n)[:count]] = np.nan
+    seq = torch.tensor(lens, dtype=torch.int32, device=dev)
+    pt = rng.permutation(len(lens) * (max(lens) // 64 + 1)).astype(np.int32).reshape(len(lens), -1)
+    for table in (None, pt):
+        got = ops.topk(torch.from_numpy(x).to(dev), seq, k,
+                       page_table=None if table is None else torch.from_numpy(table).to(dev))
+        assert np.array_equal(got.cpu().numpy(), O.topk_select(x, np.array(lens), k, page_table=table))
+    assert _lib.sync_timeouts() == 0
+
+
+@pytest.mark.parametrize("lens,k", [([4133], 2048), ([8192], 512), ([3000, 6000], 1024), ([4133] * 9, 2048)])
+def test_layers_of_nan_scores(dev, lens, k):
+    from lagged_indexer_dsa_amd import _lib
+    from lagged_indexer_dsa_amd import synthetic as S
+
+    _lib.sync_timeouts(reset=True)
+    pt, num_pages = S.make_page_table(lens, seed=71, device=dev)
+    L = S.make_decode_layer(lens, seed=72, device=dev, page_table=pt, num_pages=num_pages, topk=k)
+    scales = L.index_k[:, 8192:].view(torch.float32)  # a NaN key scale: a NaN score
+    g = torch.Generator().manual_seed(73)
+    for b, n in enumerate(lens):
+        p = torch.randperm(n, generator=g)[:k + (n - k) // 2].to(dev)
+        scales[pt[b].long()[p // 64], p % 64] = float("nan")
+    att = S.random_selection(lens, k, pt, seed=74, device=dev)
+    for attend in (att, None):  # the fused launch; scan + select, then an attention over no key
+        L.next_idx.fill_(-7)
+        L.run(attend_idx=attend)
+        torch.cuda.synchronize()
+        assert bool((L.next_idx == -1).all())
+        if attend is None:
+            assert bool((L.out == 0).all())
+    assert _lib.sync_timeouts() == 0
