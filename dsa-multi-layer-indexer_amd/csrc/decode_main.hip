@@ -509,20 +509,19 @@ struct ScanShared {
 constexpr int kCoopKeys = 16384;     // positions per workgroup
 constexpr int kCoopMaxBlocks = 256;  // workgroups per row
 constexpr int kPubHdr = 4;           // list header: count, bound key, finite count, max key
-constexpr int kCoopCand = 1024;      // threshold-bin candidates resolved by rank counting
+constexpr int kCoopCand = 256;       // sub-bin counters, then the threshold bin's candidates (at most kWave)
 constexpr int kEmitRegs = 8;         // emit: entries per thread read into registers at once
 struct CoopShared {
   ScanShared scan;
   alignas(16) uint32_t keys[kCoopKeys];
   uint16_t lpos[kPubWords];  // the published entries: own position index
   uint32_t wave_tmp[4 * kMainWaves];
-  uint32_t res[4];
   uint32_t misc[4];
   uint32_t sense[kNumSync];
   alignas(16) uint32_t ck[kCoopCand];  // threshold-bin candidates: key, union entry index
-  uint32_t ce[kCoopCand];
+  uint32_t ce[kWave];
   uint32_t wstat[2 * kMainWaves];  // per wave, from the scan: finite keys, largest key
-  uint32_t pred[2 * kMainWaves];   // per wave: union counts of pass 2
+  uint32_t pred[2 * kMainWaves];   // per wave: union counts of pass 2, ties before the own list
 };
 
 static_assert(sizeof(CoopShared) <= 160 * 1024, "the cooperative select's LDS must fit one CU");
@@ -1109,25 +1108,26 @@ __device__ __forceinline__ void coop_select(CoopShared& cs, unsigned char* smem,
       T1 = th.bin;                   // == (t* - lo) >> sh
       above = th.above;
       nbin = th.cnt;
-      // A bin of more than one wave's keys is split again, 2048 ways.  Short
-      // rows need it: their lists hold every key, so the window runs from the
-      // most negative score, its bins are a quarter of an exponent wide and the
-      // threshold's holds hundreds of keys, each of which rank counting below
-      // compared with every other (a layer of 4133 tokens 19.2 us, split
-      // 14.8; four such rows 27.3, 17.5; 131072 tokens, where the first
-      // window is enough, 14.9 and 14.8).
+      // A bin of more than one wave's keys is split again, 2048 ways, until
+      // it holds no more or a single key value (sh == 0).  Short rows need
+      // it: their lists hold every key, so the window runs from the most
+      // negative score, its bins are a quarter of an exponent wide and the
+      // threshold's holds hundreds of keys (a layer of 4133 tokens 14.8 us;
+      // comparing each of the bin's keys with every other 19.2; four such
+      // rows 17.5 and 27.3; 131072 tokens, where the first window is enough,
+      // 14.8 and 14.9).
       while (ok && nbin > (uint32_t)kWave && sh > 0) {  // uniform
-        const int width = sh;
         lo += T1 << sh;
+        // the bin's last key less lo; NaN's bin ends at 2^32, and a larger
+        // span would take in the lists' zero padding, which wraps
+        const uint32_t span = min((1u << sh) - 1u, 0xffffffffu - lo);
         sh = max(0, sh - 11);
         __syncthreads();
         for (int i = t; i < kUnionWords / 4; i += kMainThreads)
           reinterpret_cast<uint4*>(hist)[i] = make_uint4(0, 0, 0, 0);
         __syncthreads();
-        // (w >= lo: NaN's bin begins within a bin's width of 2^32, where w - lo
-        // of the lists' zero padding would wrap into it)
-        for_mine([&](uint32_t w, uint32_t) {
-          if (w >= lo && (w - lo) >> width == 0u) atomicAdd(&hist[union_slot((w - lo) >> sh)], 1u);
+        for_mine([&](uint32_t w, uint32_t) {  // (a key below lo wraps past the span)
+          if (w - lo <= span) atomicAdd(&hist[union_slot((w - lo) >> sh)], 1u);
         });
         __syncthreads();
         const BinThreshold ts = wave_threshold_sum<kUnionGroup, kUnionStride>(hist, (uint32_t)K - above);
@@ -1172,7 +1172,14 @@ __device__ __forceinline__ void coop_select(CoopShared& cs, unsigned char* smem,
       ax += before ? gj : 0u;
     }
     dbg_stamp(dbk, 13);
-    if (__ballot(cmask != 0)) {  // rare: most waves hold no candidate
+    if (nbin > (uint32_t)kWave) {  // uniform: the bin is one key value, its entries ties
+      uint32_t tb = 0;
+#pragma unroll
+      for (int j = 0; j < kU; ++j)
+        if (4u * (uint32_t)(t + j * kMainThreads) < mine0) tb += (uint32_t)__popc((cmask >> (4 * j)) & 15u);
+      tb = wave_reduce<0>(tb);
+      if (lane == 0) cs.pred[kMainWaves + wv] = tb;
+    } else if (__ballot(cmask != 0)) {  // rare: most waves hold no candidate
       for (uint32_t m = cmask; m; m &= m - 1u) {
         const int b = __builtin_ctz(m);
         const int j = b >> 2, c = b & 3;
@@ -1182,7 +1189,7 @@ __device__ __forceinline__ void coop_select(CoopShared& cs, unsigned char* smem,
         for (int jj = 0; jj < kU; ++jj)
           if (jj == j) w = c == 0 ? u[jj].x : (c == 1 ? u[jj].y : (c == 2 ? u[jj].z : u[jj].w));
         const uint32_t slot = atomicAdd(&cs.misc[1], 1u);
-        if (slot < (uint32_t)kCoopCand) {
+        if (slot < (uint32_t)kWave) {  // < nbin by construction
           cs.ck[slot] = w;
           cs.ce[slot] = e;
         }
@@ -1202,7 +1209,7 @@ __device__ __forceinline__ void coop_select(CoopShared& cs, unsigned char* smem,
       sel_before += v & 0xffffu;
       sel_above += v >> 16;
     }
-    const uint32_t nc = nbin;                   // == the candidates collected
+    const uint32_t nc = nbin;                   // up to kWave: the candidates collected
     // (value slot 27 holds the bound path)
     const uint32_t need = (uint32_t)K - above;  // 1 <= need <= nc
     if (nc <= (uint32_t)kWave) {
@@ -1230,72 +1237,11 @@ __device__ __forceinline__ void coop_select(CoopShared& cs, unsigned char* smem,
       ties_before = (uint32_t)__popcll(__ballot(tie && before));
       sel_above += (uint32_t)__popcll(__ballot(g));
     } else {
-      if (nc <= (uint32_t)kCoopCand) {
-        // rank counting in 16-byte broadcast reads: pad the last uint4 with
-        // 0 (below every candidate)
-        if (t < 3 && nc + (uint32_t)t < (uint32_t)kCoopCand) cs.ck[nc + t] = 0u;
-        __syncthreads();
-        const uint4* c4 = reinterpret_cast<const uint4*>(cs.ck);
-        const int nq = ((int)nc + 3) >> 2;
-        for (uint32_t j = t; j < nc; j += kMainThreads) {
-          const uint32_t c = cs.ck[j];
-          uint32_t gtc = 0, gec = 0;
-#pragma unroll 4
-          for (int q = 0; q < nq; ++q) {
-            const uint4 x = c4[q];
-            gtc += (x.x > c ? 1u : 0u) + (x.y > c ? 1u : 0u) + (x.z > c ? 1u : 0u) + (x.w > c ? 1u : 0u);
-            gec += (x.x >= c ? 1u : 0u) + (x.y >= c ? 1u : 0u) + (x.z >= c ? 1u : 0u) + (x.w >= c ? 1u : 0u);
-          }
-          if (gtc < need && need <= gec) {
-            cs.res[0] = c;
-            cs.res[1] = need - gtc;
-          }
-        }
-        __syncthreads();
-        tstar = cs.res[0];
-        need3 = cs.res[1];
-      } else {
-        // many keys share T1's bin: refine its low sh bits, <= 10 per level
-        uint32_t* hist = cs.scan.hist;
-        uint32_t prefix = T1, nd = need;
-        int s2 = sh;
-        while (s2 > 0) {
-          const int sub = min(10, s2);
-          s2 -= sub;
-          for (int i = t; i < kNB2; i += kMainThreads) hist[i] = 0u;
-          __syncthreads();
-          const int hs = s2 + sub;
-          for_mine([&](uint32_t w, uint32_t) {
-            if (w >= lo && ((w - lo) >> hs) == prefix) atomicAdd(&hist[((w - lo) >> s2) & ((1u << sub) - 1u)], 1u);
-          });
-          __syncthreads();
-          find_threshold_fixed<kNB2, kMainThreads>(hist, nd, cs.wave_tmp, cs.res);
-          prefix = (prefix << sub) | cs.res[0];
-          nd -= cs.res[1];
-        }
-        tstar = lo + prefix;
-        need3 = nd;
-      }
-      // the bin-T1 keys' share (keys above the bin were counted in pass 2)
-      uint4 acc = make_uint4(0, 0, 0, 0);
-      const auto count = [&](uint32_t w, uint32_t e) {
-        const bool g = w > tstar && key_is_finite(w);
-        const bool before = e < mine0;
-        acc.x += (g && before) ? 1u : 0u;
-        acc.y += (w == tstar && before) ? 1u : 0u;
-        acc.z += g ? 1u : 0u;
-      };
-      if (nc <= (uint32_t)kCoopCand) {
-        for (uint32_t j = t; j < nc; j += kMainThreads) count(cs.ck[j], cs.ce[j]);
-      } else {
-        for_mine([&](uint32_t w, uint32_t e) {
-          if (w >= lo && ((w - lo) >> sh) == T1) count(w, e);
-        });
-      }
-      const uint4 r = block_reduce4<0, 0, 0, 0>(acc, cs.wave_tmp);
-      sel_before += r.x;
-      ties_before = r.y;
-      sel_above += r.z;
+      // equal keys only: all of them candidates, no rank to find
+      tstar = bot;
+      need3 = need;
+#pragma unroll
+      for (int w = 0; w < kMainWaves; ++w) ties_before += cs.pred[kMainWaves + w];
     }
     }  // the lists decide
     dbg_stamp(dbk, 15);

@@ -123,36 +123,6 @@ __device__ __forceinline__ void find_threshold(const uint32_t* hist, int nbins, 
   __syncthreads();
 }
 
-// find_threshold for a compile-time NBINS / NT (>= 1 bin per thread),
-// every loop unrolled so the LDS reads are in flight together; also writes
-// the histogram's total to res[2] (res: 3 words).
-template <int NBINS, int NT>
-__device__ __forceinline__ void find_threshold_fixed(const uint32_t* hist, uint32_t need, uint32_t* wave_tmp,
-                                                     uint32_t* res) {
-  constexpr int kPer = NBINS / NT;
-  static_assert(kPer >= 1 && NBINS % NT == 0, "bins per thread");
-  const int hi = NBINS - (int)threadIdx.x * kPer;
-  uint32_t h[kPer];
-  uint32_t local = 0;
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    h[i] = hist[hi - 1 - i];
-    local += h[i];
-  }
-  uint32_t total;
-  uint32_t acc = block_exclusive_scan(local, wave_tmp, &total);
-  if (threadIdx.x == 0) res[2] = total;
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    if (acc < need && acc + h[i] >= need) {
-      res[0] = (uint32_t)(hi - 1 - i);
-      res[1] = acc;
-    }
-    acc += h[i];
-  }
-  __syncthreads();
-}
-
 // dst[0..n) = src[0..n) for n 32-bit words, with every load of the block
 // issued before any LDS store (PER uint4 per thread covers n <= PER*4*blockDim).
 // Both pointers 16-byte aligned; the tail (n % 4) is copied word by word.

@@ -119,3 +119,31 @@ def test_layers_of_nan_scores(dev, lens, k):
         if attend is None:
             assert bool((L.out == 0).all())
     assert _lib.sync_timeouts() == 0
+
+
+# A threshold bin of more than a wave's equal scores: the split ends at one
+# key value, whose entries are taken lowest position first.
+@pytest.mark.parametrize("ties", [63, 64, 65, 130, 1024, 1500])
+@pytest.mark.parametrize("lens,k", [([2600], 2048), ([4133], 1024), ([6000], 2048), ([20000], 2048), ([131072], 2048),
+                                    ([4133, 2600, 3000], 2048)])
+def test_ties_at_the_threshold(dev, lens, k, ties):
+    from lagged_indexer_dsa_amd import _lib, ops
+
+    _lib.sync_timeouts(reset=True)
+    rng = np.random.default_rng(ties + k + sum(lens))
+    x = rng.standard_normal((len(lens), max(lens))).astype(np.float32)
+    for r, n in enumerate(lens):
+        # k - ties // 3 scores above the tied ones, the others below
+        order = np.argsort(-x[r, :n], kind="stable")
+        top = k - ties // 3
+        tied = rng.permutation(order[top:])[:ties]
+        v = x[r, order[top]]
+        x[r, order[top:]] = np.minimum(x[r, order[top:]], np.nextafter(v, np.float32(-np.inf)))
+        x[r, tied] = v
+    seq = torch.tensor(lens, dtype=torch.int32, device=dev)
+    pt = rng.permutation(len(lens) * (max(lens) // 64 + 1)).astype(np.int32).reshape(len(lens), -1)
+    for table in (None, pt):
+        got = ops.topk(torch.from_numpy(x).to(dev), seq, k,
+                       page_table=None if table is None else torch.from_numpy(table).to(dev))
+        assert np.array_equal(got.cpu().numpy(), O.topk_select(x, np.array(lens), k, page_table=table))
+    assert _lib.sync_timeouts() == 0
