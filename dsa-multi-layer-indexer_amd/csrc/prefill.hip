@@ -34,10 +34,13 @@ constexpr int kPfLoads = kPfKeys * kPfRowChunks / kPfThreads; // 9 direct-to-LDS
 static_assert(kPfLoads * kPfThreads == kPfKeys * kPfRowChunks, "whole loads");
 
 constexpr float kPfRise = 32.f;
+// A wave takes the second bf16 term of a tile's probabilities too when one of
+// its rows has a probability above this share of the row's sum so far.
+constexpr float kPfSecond = 1.f / 24.f;
 
 struct PrefillArgs {
   const uint16_t* q;     // [B, S*H, 576] bf16
-  const uint16_t* keys;  // [B, Tpad, 576] bf16, Tpad = T rounded up to 64
+  const uint16_t* keys;  // [B, Tpad, 576] bf16, Tpad = T rounded up to 32
   const uint32_t* mask;  // MASK: [B*S, Tpad / 32], bit j of a query: it attends key j
   uint16_t* out;         // [B, S*H, 512] bf16
   float* part_o;         // nsplit > 1: [nsplit][B*S*H][512]
@@ -95,11 +98,12 @@ __device__ __forceinline__ float half_swap_sum(float v) {
 // 32 rows go from memory straight to LDS, two buffers, the next tile in
 // flight while this one is used.
 //
-// Bound by the matrix cores and the LDS reads that feed them: 2999 causal
-// queries of 16 heads in 182 us (860 TFLOP/s; a library product of 8192^3
-// reaches 1218 here), 1024 over 8192 keys in 267 us; a decode row per query
-// took 1115 us and 2.5 ms of workspace fills.  Fragments read 4, 6, 8 and 10
-// steps ahead: 193, 184, 182 and 210 us.
+// Bound by the matrix cores and the LDS reads that feed them: a call with 2999
+// causal queries of 16 heads takes 220 us (156 GFLOP and the second terms of
+// the probabilities; a library product of 8192^3 reaches 1218 TFLOP/s here);
+// a decode row per query took 1115 us and 2.5 ms of workspace fills.
+// Fragments read 4, 6, 8 and 10 steps ahead, with one term: 193, 184, 182 and
+// 210 us of kernel.
 template <bool MASK>
 __global__ __launch_bounds__(kPfThreads, 1) void prefill_attention_kernel(const PrefillArgs A) {
   __shared__ __align__(16) uint16_t kb[2 * kPfKeys * DSA_QK_DIM];
@@ -202,7 +206,7 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_attention_kernel(const 
 #pragma unroll
     for (int e = 0; e < 16; ++e) s[0][e] += s[1][e];
     // scores in the log2 domain; keys at or past the row's limit: -inf.
-    // Element i of block c is key 32c + 8 (i / 4) + 4h + (i % 4).
+    // Element i is the tile's key 8 (i / 4) + 4h + (i % 4).
     const int k0 = tl * kPfKeys;
     const bool edge = k0 + kPfKeys > kfull;  // uniform
     float tmax = -INFINITY;
@@ -230,8 +234,9 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_attention_kernel(const 
     uint32_t pk[8];
 #pragma unroll
     for (int i = 0; i < 16; i += 2) {
-      const float p0 = __builtin_amdgcn_exp2f(s[0][i] - mr), p1 = __builtin_amdgcn_exp2f(s[0][i + 1] - mr);
-      pk[i >> 1] = pack_bf16x2(p0, p1);
+      s[0][i] = __builtin_amdgcn_exp2f(s[0][i] - mr);
+      s[0][i + 1] = __builtin_amdgcn_exp2f(s[0][i + 1] - mr);
+      pk[i >> 1] = pack_bf16x2(s[0][i], s[0][i + 1]);
       // the sum of the rounded probabilities, the ones PV multiplies: the
       // weights then add up to one (0-1.3% less error than the unrounded sum)
       l = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, pk[i >> 1]), __builtin_bit_cast(v2bf, 0x3f803f80u),
@@ -248,15 +253,41 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_attention_kernel(const 
       __builtin_memcpy(&vf.z, &hi, 8);
       return vf;
     };
-    uint4 vf[kPfDepth];
+    // Probabilities are rounded to bf16, and a row's largest is 1 exactly only
+    // when it lies in the row's first tile: with one term the error against
+    // 64 bits was up to 4% above that of a softmax about the true maximum.
+    // Tiles that hold much of a row's weight take what the rounding left in a
+    // second product, which more than makes up for it (kPfSecond):
+    // (error, and us a call)        one term      1/16       1/24       1/32     always
+    //   2999 queries            0.00200 205  .00177 221  .00173 220  .00171 227  .00162 253
+    //   1024 over 2999 keys     0.00195 160  .00190 170  .00186 176  .00183 179  .00166 185
+    //   512 over 16384          0.00173 312  .00172 320  .00172 327  .00172 331  .00166 381
+    //   1024 over 4096, masked  0.00198 170  .00192 189  .00188 198  .00184 204  .00166 204
+    // (a decode row a query, rounded about its running maximum: 0.00196,
+    // 0.00192, 0.00172 and 0.00194).
+    const bool two = __ballot(__builtin_amdgcn_exp2f(tmax - mr) > kPfSecond * half_swap_sum(l)) != 0;  // uniform
+    // one copy of the products in the code: unrolled, or as two branches, the
+    // accumulators cross the vector file at the join and spill
+#pragma nounroll
+    for (int term = 0;; ++term) {
+      uint4 vf[kPfDepth];
 #pragma unroll
-    for (int i = 0; i < kPfDepth; ++i) vf[i] = v_frag(i);
+      for (int i = 0; i < kPfDepth; ++i) vf[i] = v_frag(i);
 #pragma unroll
-    for (int i = 0; i < 32; ++i) {
-      const uint32_t* pr = &pk[4 * (i >> 4)];
-      const v8bf pb = as_bf8(make_uint4(pr[0], pr[1], pr[2], pr[3]));
-      o[i & 15] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(vf[i % kPfDepth]), pb, o[i & 15], 0, 0, 0);
-      if (i + kPfDepth < 32) vf[i % kPfDepth] = v_frag(i + kPfDepth);
+      for (int i = 0; i < 32; ++i) {
+        const uint32_t* pr = &pk[4 * (i >> 4)];
+        const v8bf pb = as_bf8(make_uint4(pr[0], pr[1], pr[2], pr[3]));
+        o[i & 15] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(vf[i % kPfDepth]), pb, o[i & 15], 0, 0, 0);
+        if (i + kPfDepth < 32) vf[i % kPfDepth] = v_frag(i + kPfDepth);
+      }
+      if (term || !two) break;
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) {
+        pk[i >> 1] = pack_bf16x2(s[0][i] - __uint_as_float(pk[i >> 1] << 16),
+                                 s[0][i + 1] - __uint_as_float(pk[i >> 1] & 0xffff0000u));
+        l = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, pk[i >> 1]), __builtin_bit_cast(v2bf, 0x3f803f80u),
+                                            l, false);
+      }
     }
   };
 

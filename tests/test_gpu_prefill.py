@@ -167,3 +167,40 @@ def test_pack_latent_rows_bytes(dev, dt):
     for src in (x, off, wide[..., 7:583]):
         got = ops.pack_latent_rows(src, 40).reshape(2, 40, 656)
         assert torch.equal(got[:, :37], want) and not got[:, 37:].any()
+
+
+@pytest.mark.parametrize("S,T,n,scale", [(1000, 1000, 0, 1.0), (2999, 2999, 0, 1.0), (64, 2999, 0, 1.0),
+                                         (512, 4096, 0, 1.0), (700, 700, 0, 3.0), (600, 1200, 512, 1.0),
+                                         (512, 4096, 2048, 1.0)])
+def test_error_is_that_of_a_softmax_about_the_maximum(dev, S, T, n, scale):
+    """The error against 64 bits is no larger than that of one bf16 term a
+    probability about the row's true maximum (1 exactly for the largest),
+    normalised by the sum of the rounded ones, and the rounding of the output."""
+    from lagged_indexer_dsa_amd import attention_core as ac
+
+    print(f"[prefill] error S={S} T={T} n={n}", flush=True)
+    H = 16
+    g = torch.Generator(device=dev).manual_seed(T + S)
+    q = (scale * torch.randn(1, S, H, 576, generator=g, device=dev)).to(torch.bfloat16)
+    kv = torch.randn(1, T, 576, generator=g, device=dev).to(torch.bfloat16)
+    mask = _causal(S, T, dev)
+    if n:
+        idx = torch.rand(1, S, T, generator=g, device=dev).masked_fill(~mask, -1.0).topk(n, -1).indices
+        got = ac.sparse_mla_core(q, kv, idx, 512)
+        mask = mask & torch.zeros(1, S, T, dtype=torch.bool, device=dev).scatter_(2, idx, True)[0]
+    else:
+        got = ac.dense_mla_core(q, kv, 512)
+    keys = _values(kv).to(dev)[0]
+    err, about_max, size = 0.0, 0.0, 0.0
+    for s0 in range(0, S, 128):
+        s = torch.matmul(q[0, s0:s0 + 128].double(), keys.t().contiguous()) * 576 ** -0.5
+        s = s.masked_fill(~mask[s0:s0 + 128, None], float("-inf"))
+        p = torch.exp(s - s.amax(-1, keepdim=True))
+        ref = torch.matmul(p, keys[:, :512].contiguous()) / p.sum(-1, keepdim=True)
+        p = p.to(torch.bfloat16).double()
+        one = (torch.matmul(p, keys[:, :512].contiguous()) / p.sum(-1, keepdim=True)).to(torch.bfloat16).double()
+        err += float((got[0, s0:s0 + 128].double() - ref).square().sum())
+        about_max += float((one - ref).square().sum())
+        size += float(ref.square().sum())
+    print(f"[prefill] error {(err / size) ** 0.5:.6f}, about the maximum {(about_max / size) ** 0.5:.6f}", flush=True)
+    assert err <= about_max
