@@ -132,6 +132,8 @@ def select_rows(scores: torch.Tensor, k: int, pad_value: int) -> torch.Tensor | 
     """:func:`topk` with sorted=True over whole rows, as int64 and in one
     launch; None for the shapes the row kernel does not take."""
     _dev(scores)
+    if scores.dim() != 2 or scores.dtype != torch.float32:
+        raise RuntimeError("scores must be [B, slab] float32")
     B, slab = scores.shape
     if not _lib.load().dsa_select_rows_supported(B, slab, k):
         return None
@@ -250,6 +252,11 @@ def _kernel_input(x: torch.Tensor) -> torch.Tensor:
     return x if x.data_ptr() % 16 == 0 else x.clone()
 
 
+def _need_kv(kv: torch.Tensor) -> None:
+    if kv.dim() != 3 or kv.shape[2] != QK_DIM:
+        raise RuntimeError(f"kv must be [B, T, 576], got {tuple(kv.shape)}")
+
+
 def _pack_source(kv: torch.Tensor) -> torch.Tensor:
     """kv [B, T, 576] as the pack kernels read it (rope rounded to bf16 once)."""
     if kv.dtype not in _PACK_DTYPES:
@@ -264,7 +271,13 @@ def prefill_logits(q: torch.Tensor, k: torch.Tensor, w: torch.Tensor) -> torch.T
     k [B, T, 128], quantised per row inside.  Reference: attention_core.py:27-49."""
     q, k, w = _kernel_input(q), _kernel_input(k), _kernel_input(w)
     _dev(q, k, w)
+    if q.dim() != 4 or q.shape[3] != INDEX_DIM:
+        raise RuntimeError(f"q must be [B, S, H, 128], got {tuple(q.shape)}")
     B, S, H, _ = q.shape
+    if k.dim() != 3 or k.shape[0] != B or k.shape[2] != INDEX_DIM:
+        raise RuntimeError(f"k must be [{B}, T, 128], got {tuple(k.shape)}")
+    if w.shape != (B, S, H):
+        raise RuntimeError(f"w must be {(B, S, H)}, got {tuple(w.shape)}")
     T = k.shape[1]
     ws = torch.empty(_lib.load().dsa_prefill_logits_workspace_bytes(B, S, H, T), dtype=torch.uint8, device=q.device)
     out = torch.empty(B, S, T, dtype=torch.float32, device=q.device)
@@ -276,9 +289,12 @@ def prefill_logits(q: torch.Tensor, k: torch.Tensor, w: torch.Tensor) -> torch.T
 def pack_latent_rows(kv: torch.Tensor, row_stride: int) -> torch.Tensor:
     """kv [B, T, 576] -> 656-byte fp8 rows [B * row_stride, 656] (rows past T
     of a request zero)."""
+    _need_kv(kv)
     kv = _pack_source(kv)
     _dev(kv)
     B, T, _ = kv.shape
+    if row_stride < T:
+        raise RuntimeError(f"row_stride {row_stride} below the {T} rows of a request")
     rows = torch.empty(B * row_stride, LATENT_ROW_BYTES, dtype=torch.uint8, device=kv.device)
     _lib.call("dsa_pack_latent_rows", kv.data_ptr(), _PACK_DTYPES[kv.dtype], B, T, row_stride, rows.data_ptr(),
               _stream())
@@ -291,6 +307,8 @@ def selection_set(idx: torch.Tensor, T: int, as_bits: bool) -> torch.Tensor:
     row, or the KV slots b * T + position ascending, then -1 [B * S, n]."""
     idx = idx.contiguous()
     _dev(idx)
+    if idx.dim() != 3 or idx.dtype not in (torch.int32, torch.int64):
+        raise RuntimeError(f"idx must be [B, S, n] int32 or int64, got {idx.dtype} {tuple(idx.shape)}")
     B, S, n = idx.shape
     lib = _lib.load()
     if as_bits:
@@ -307,17 +325,23 @@ def prefill_attention(q: torch.Tensor, kv: torch.Tensor, bits: torch.Tensor | No
     """q [B, S, H, 576] bf16 over kv [B, T, 576]: query row s of S attends keys
     0 .. T - S + s, or those of its bitmap (:func:`selection_set`) ->
     [B, S, H, 512] bf16.  Reference: attention_core.py:121-160."""
+    _need_kv(kv)
     kv = _pack_source(kv)
     _dev(q, kv)
-    if q.dtype != torch.bfloat16:
-        raise RuntimeError("q must be bfloat16")
+    if q.dim() != 4 or q.shape[3] != QK_DIM or q.dtype != torch.bfloat16:
+        raise RuntimeError("q must be [B, S, H, 576] bfloat16")
     B, S, H, _ = q.shape
+    if kv.shape[0] != B:
+        raise RuntimeError(f"kv holds {kv.shape[0]} requests, q {B}")
     T = kv.shape[1]
     lib = _lib.load()
     keys = torch.empty(lib.dsa_prefill_keys_bytes(B, T), dtype=torch.uint8, device=q.device)
     ws = torch.empty(lib.dsa_prefill_workspace_bytes(B, S, H, T), dtype=torch.uint8, device=q.device)
     out = torch.empty(B, S, H, LATENT_DIM, dtype=torch.bfloat16, device=q.device)
     if bits is not None:
+        _dev(bits)
+        if bits.dtype != torch.int32:
+            raise RuntimeError("bits must be int32")
         _need_bytes("bits", bits, lib.dsa_selection_bits_bytes(B * S, T))
     st = _stream()
     _lib.call("dsa_pack_prefill_keys", kv.data_ptr(), _PACK_DTYPES[kv.dtype], B, T, keys.data_ptr(), st)
