@@ -130,9 +130,12 @@ __global__ __launch_bounds__(kSelThreads) void select_rows_kernel(const float* _
     if (i < (int)ntop || i >= (int)(ntop + need)) o[i] = (OUT)pad;
   if (need == 0) return;  // uniform
 
-  const float lo = key_value(st.x), range = key_value(st.y) - lo;
+  float lo = key_value(st.x);
+  const float range = key_value(st.y) - lo;
   float scale = (float)(kSelBins - 1) / range;
-  if (!(range > 0.f) || !(scale > 0.f) || !(scale < INFINITY)) scale = 0.f;  // (range inf, 0 or denormal)
+  // range inf, 0 or denormal: one bin, and lo 0 so that (x - lo) * scale is 0
+  // (with an infinite difference it would be NaN, which no integer stands for)
+  if (!(range > 0.f) || !(scale > 0.f) || !(scale < INFINITY)) scale = lo = 0.f;
   const auto bin_of = [&](uint32_t x) { return min((int)((key_value(x) - lo) * scale), kSelBins - 1); };
   each([&](uint32_t x, int, int j) {
     if (key_is_finite(x)) {

@@ -80,3 +80,21 @@ def test_few_very_long_rows_take_the_slice_kernels(dev):
     assert ops.select_rows(torch.from_numpy(x).to(dev), 2048, n) is None
     ref = O.topk_select(x, np.full(2, n, dtype=np.int32), 2048, sorted_=True, pad=n)
     assert np.array_equal(ac.select_topk(torch.from_numpy(x).to(dev)[None], 2048)[0].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("n,k,finite", [(2048, 64, 2), (2049, 300, 100), (8192, 2048, 128), (8193, 2048, 129),
+                                        (16384, 2048, 16384), (20000, 512, 120), (20000, 512, 20000)])
+def test_rows_whose_range_overflows(dev, n, k, finite):
+    """Finite scores further apart than the largest float: one bin, of few
+    members (ranked) and of many (the radix form)."""
+    from lagged_indexer_dsa_amd import ops
+
+    rng = np.random.default_rng(n + finite)
+    x = np.full((3, n), -np.inf, dtype=np.float32)
+    for r in range(3):
+        p = rng.permutation(n)[:finite]
+        x[r, p] = rng.uniform(-3e38, 3e38, finite)
+        x[r, p[0]], x[r, p[1]] = 3.4e38, -3.4e38
+    got = ops.select_rows(torch.from_numpy(x).to(dev), k, n)
+    ref = O.topk_select(x, np.full(3, n, dtype=np.int32), k, sorted_=True, pad=n)
+    assert np.array_equal(got.cpu().numpy(), ref)
