@@ -575,6 +575,16 @@ hipError_t launch_selection_set(const void* idx, int idx64, int rows, int n, int
   const int words = selection_words(T);
   const dim3 grid((unsigned)rows), block(kSetThreads);
   const size_t lds = (size_t)words * 4;
+  // the longest context's bitmap and the slots form's sums pass 64 KB together
+  static PerDeviceOnce attr;
+  const hipError_t e = attr.run([] {
+    for (const void* f : {(const void*)selection_set_kernel<int64_t, true>, (const void*)selection_set_kernel<int64_t, false>,
+                          (const void*)selection_set_kernel<int, true>, (const void*)selection_set_kernel<int, false>})
+      if (hipError_t r = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, DSA_SELECTION_MAX_CTX / 8))
+        return r;
+    return hipSuccess;
+  });
+  if (e != hipSuccess) return e;
   const auto go = [&](auto kernel, auto* src) {
     hipLaunchKernelGGL(kernel, grid, block, lds, s, src, n, S, T, words, bits, slots);
   };

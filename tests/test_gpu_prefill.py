@@ -204,3 +204,21 @@ def test_error_is_that_of_a_softmax_about_the_maximum(dev, S, T, n, scale):
         size += float(ref.square().sum())
     print(f"[prefill] error {(err / size) ** 0.5:.6f}, about the maximum {(about_max / size) ** 0.5:.6f}", flush=True)
     assert err <= about_max
+
+
+@pytest.mark.parametrize("T", [524288, 524287, 523264])
+@pytest.mark.parametrize("itype", [torch.int64, torch.int32])
+def test_selection_set_at_the_longest_context(dev, T, itype):
+    """The bitmap fills 64 KB of LDS: first, last and middle positions, and
+    those the row does not see."""
+    from lagged_indexer_dsa_amd import ops
+
+    S = 3
+    idx = torch.tensor([0, T - 1, T - 2, T - 3, T - 4, T // 2, T, -1, 31, 32, T - 1], device=dev).to(itype)
+    idx = idx.expand(1, S, -1).contiguous()
+    bits = ops.selection_set(idx, T, True).cpu().numpy().view(np.uint32).reshape(S, -1)
+    slots = ops.selection_set(idx, T, False).cpu().numpy()
+    for s in range(S):
+        want = sorted(v for v in {0, T - 1, T - 2, T - 3, T - 4, T // 2, 31, 32} if v < T - S + s + 1)
+        assert np.flatnonzero(np.unpackbits(bits[s].view(np.uint8), bitorder="little")).tolist() == want
+        assert slots[s].tolist() == want + [-1] * (idx.shape[2] - len(want))
