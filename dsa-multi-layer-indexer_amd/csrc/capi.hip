@@ -470,6 +470,14 @@ size_t dsa_sparse_mla_workspace_bytes(int B, int H, int nsplit) {
   return dsa::attn_workspace_bytes(B, H, nsplit > 0 ? nsplit : 128);
 }
 
+size_t dsa_sparse_mla_barrier_bytes(int B, int H, int nsplit) {
+  if (dsa_sparse_mla_workspace_bytes(B, H, nsplit) == 0) return 0;
+  dsa::AttnArgs A{};
+  A.H = H;
+  A.nsplit = nsplit;
+  return dsa::mla_rows_takes(A, B) ? 0 : dsa::attn_workspace_bytes(B, H, 0);
+}
+
 int dsa_sparse_mla_decode(const void* q_bf16, const void* kv_pool, int64_t kv_rows,
                           const int32_t* idx, void* workspace, void* out_bf16, int B, int H,
                           int topk, int nsplit, float sm_scale, void* stream) {

@@ -78,6 +78,7 @@ SIGNATURES = {
     "dsa_select_rows_supported": (_i32, [_i32, _i32, _i32]),
     "dsa_select_rows": (_i32, [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _vp]),
     "dsa_sparse_mla_workspace_bytes": (ctypes.c_size_t, [_i32, _i32, _i32]),
+    "dsa_sparse_mla_barrier_bytes": (ctypes.c_size_t, [_i32, _i32, _i32]),
     "dsa_sparse_mla_decode": (_i32, [_vp, _vp, _i64, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _vp]),
     "dsa_dense_mla_decode": (_i32, [_vp, _vp, _i64, _vp, _i32, _vp, _vp, _vp, _i32, _i32, _i32, _f32, _vp]),
     "dsa_sparse_mla_decode_noalloc": (_i32, [_vp, _vp, _i64, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _vp]),

@@ -153,14 +153,15 @@ def sparse_mla_workspace(B: int, H: int, nsplit: int, device) -> torch.Tensor:
 
 def _call_workspace(B: int, H: int, nsplit: int, device) -> torch.Tensor:
     """Workspace of one call at a known split count: the barriers zeroed, the
-    partials (overwritten before they are read) not."""
+    partials (overwritten before they are read) not.  Many unsplit rows read
+    neither."""
     lib = _lib.load()
     nbytes = lib.dsa_sparse_mla_workspace_bytes(B, H, nsplit)
     if nbytes == 0:
         raise RuntimeError(f"bad sparse MLA workspace shape B={B} H={H} nsplit={nsplit}")
-    ws = torch.empty(nbytes // 4, dtype=torch.float32, device=device)
-    partials = nsplit * B * (H // 16) * 16 * (LATENT_DIM + 2)
-    ws[:ws.numel() - partials].zero_()
+    barriers = lib.dsa_sparse_mla_barrier_bytes(B, H, nsplit)
+    ws = torch.empty(nbytes // 4 if barriers else 4, dtype=torch.float32, device=device)
+    ws[:barriers // 4].zero_()
     return ws
 
 
@@ -192,12 +193,13 @@ def sparse_mla_decode(q: torch.Tensor, kv_pool: torch.Tensor, idx: torch.Tensor,
     if workspace is None:
         nsplit = _resolve_nsplit(nsplit, B, H, idx.shape[1])
         workspace = _call_workspace(B, H, nsplit, q.device)
+    else:  # sized for this nsplit (nsplit=0, the library's choice: the largest size)
+        _dev(workspace)
+        _need_bytes("sparse MLA workspace", workspace, _lib.load().dsa_sparse_mla_workspace_bytes(B, H, nsplit))
     if out is None:
         out = torch.empty(B, H, LATENT_DIM, dtype=torch.bfloat16, device=q.device)
-    _dev(workspace, out)
+    _dev(out)
     _need_shape("out", out, (B, H, LATENT_DIM), torch.bfloat16)
-    # sized for this nsplit (nsplit=0, the library's choice: the largest size)
-    _need_bytes("sparse MLA workspace", workspace, _lib.load().dsa_sparse_mla_workspace_bytes(B, H, nsplit))
     _lib.call("dsa_sparse_mla_decode", q.data_ptr(), kv_pool.data_ptr(), kv_pool.shape[0],
               idx.data_ptr(), workspace.data_ptr(), out.data_ptr(), B, H, idx.shape[1], nsplit,
               float(sm_scale), _stream())
@@ -229,11 +231,13 @@ def dense_mla_decode(q: torch.Tensor, kv_pool: torch.Tensor, page_table: torch.T
     if workspace is None:
         nsplit = _resolve_nsplit(nsplit, B, H, page_table.shape[1] * PAGE_TOKENS)
         workspace = _call_workspace(B, H, nsplit, q.device)
+    else:  # sized for this nsplit (nsplit=0, the library's choice: the largest size)
+        _dev(workspace)
+        _need_bytes("sparse MLA workspace", workspace, _lib.load().dsa_sparse_mla_workspace_bytes(B, H, nsplit))
     if out is None:
         out = torch.empty(B, H, LATENT_DIM, dtype=torch.bfloat16, device=q.device)
-    _dev(workspace, out)
+    _dev(out)
     _need_shape("out", out, (B, H, LATENT_DIM), torch.bfloat16)
-    _need_bytes("sparse MLA workspace", workspace, _lib.load().dsa_sparse_mla_workspace_bytes(B, H, nsplit))
     _lib.call("dsa_dense_mla_decode", q.data_ptr(), kv_pool.data_ptr(), kv_pool.shape[0], page_table.data_ptr(),
               page_table.shape[1], seq_lens.data_ptr(), workspace.data_ptr(), out.data_ptr(), B, H, nsplit,
               float(sm_scale), _stream())

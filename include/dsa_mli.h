@@ -192,10 +192,14 @@ int dsa_select_rows(const float* scores, const int32_t* seq_lens, int64_t* out_i
  *   out       [B, H, 512] bf16
  * H must be a multiple of 16; 1 <= nsplit <= 128 (nsplit=0: automatic, and
  * a workspace sized with nsplit=0 fits any nsplit).
+ * dsa_sparse_mla_barrier_bytes: how many bytes at the workspace's start hold
+ * the barriers, the only part that needs the zero-fill; 0 where the call with
+ * this split count (>= 1) reads no workspace (many unsplit rows).
  * Replaces: hp_attention_block + combine (K:1312-1666, K:996-1045) and
  * ref_sparse_mla (K:2950-2966); CPU semantics attention_core.py:94-146.
  */
 size_t dsa_sparse_mla_workspace_bytes(int B, int H, int nsplit);
+size_t dsa_sparse_mla_barrier_bytes(int B, int H, int nsplit);
 int dsa_sparse_mla_decode(const void* q_bf16, const void* kv_pool,
                           int64_t kv_rows, const int32_t* idx, void* workspace,
                           void* out_bf16, int B, int H, int topk, int nsplit,

@@ -111,6 +111,12 @@ def test_mla_contract_and_workspace(lib):
     assert ws(2, 32, 8) == (4 * sync + 2 * 2 * 8 * 16 * 514) * 4
     assert ws(1, 16, 0) == ws(1, 16, 128)
     assert ws(1, 15, 8) == 0
+    barriers = lib.dsa_sparse_mla_barrier_bytes                  # the part to zero
+    assert barriers(1, 16, 32) == barriers(1, 16, 1) == barriers(1, 16, 0) == sync * 4
+    assert barriers(2, 32, 8) == 4 * sync * 4
+    assert barriers(300, 16, 2) == 300 * sync * 4
+    assert barriers(300, 16, 1) == 0                             # unsplit rows: no workspace read
+    assert barriers(1, 15, 8) == 0
 
 
 def test_mli_contract(lib):

@@ -122,3 +122,31 @@ def test_workspace_shared_across_split_counts(dev):
         torch.cuda.synchronize()
         assert torch.equal(got.view(torch.int16), ref.view(torch.int16)), ns
     assert lib.dsa_internal_group_wait_timeouts(1) == 0
+
+
+@pytest.mark.parametrize("B,H,ns", [(1, 16, 1), (3, 32, 2), (2, 64, 8), (1, 16, 0), (128, 16, 1), (129, 16, 1),
+                                    (129, 16, 0), (65, 32, 2)])
+def test_call_workspace_in_used_memory(dev, B, H, ns):
+    """A call without a workspace takes memory that earlier tensors left
+    dirty: equal to the call with a zeroed workspace, sparse and dense."""
+    from lagged_indexer_dsa_amd import _lib, ops
+
+    lib = _lib.load()
+    lib.dsa_internal_group_wait_timeouts(1)
+    case = C.latent_case(78, 700, B, H, 512)
+    q = C.q_bf16_dev(case["q"], dev)
+    rows = torch.from_numpy(case["rows"]).to(dev)
+    idx = torch.from_numpy(case["idx"]).to(dev)
+    pt = torch.arange(8, dtype=torch.int32, device=dev).repeat(B, 1)
+    lens = torch.full((B,), 500, dtype=torch.int32, device=dev)
+    dirty = [torch.full((lib.dsa_sparse_mla_workspace_bytes(B, H, n),), 0xff, dtype=torch.uint8, device=dev)
+             for n in (1, 2, 8)]
+    del dirty
+    got = ops.sparse_mla_decode(q, rows, idx, nsplit=ns), ops.dense_mla_decode(q, rows, pt, lens, nsplit=ns)
+    ws = ops.sparse_mla_workspace(B, H, 0, dev)
+    ref = (ops.sparse_mla_decode(q, rows, idx, nsplit=ns, workspace=ws),
+           ops.dense_mla_decode(q, rows, pt, lens, nsplit=ns, workspace=ws))
+    torch.cuda.synchronize()
+    for g, r in zip(got, ref):
+        assert torch.equal(g.view(torch.int16), r.view(torch.int16))
+    assert lib.dsa_internal_group_wait_timeouts(1) == 0
