@@ -45,6 +45,11 @@ def _gpu(*ts: torch.Tensor) -> None:
             raise RuntimeError("lagged_indexer_dsa_amd.attention_core runs on GPU (HIP) tensors only")
 
 
+def _need_rows(rows: int) -> None:
+    if not 1 <= rows <= 65535:
+        raise RuntimeError(f"B * S must be in [1, 65535] (got {rows})")
+
+
 def pad_index(seq_len_kv: int) -> int:
     """The out-of-range index sentinel: ``S_kv`` (attention_core.py:21-23)."""
     return seq_len_kv
@@ -71,7 +76,10 @@ def indexer_logits(index_q: torch.Tensor, index_k: torch.Tensor, weights: torch.
     if D != INDEX_DIM:
         raise ValueError(f"the fp8 indexer contracts D = {INDEX_DIM}, got {D}")
     _gpu(index_q, index_k, weights)
-    if index_k.shape[1] == 0:  # no key
+    if index_k.shape[1] == 0:  # no key: nothing to launch, the other limits hold
+        _need_rows(B * S)
+        if H not in (16, 32, 48, 64):
+            raise RuntimeError(f"index_n_heads must be 16, 32, 48 or 64 (got {H})")
         return torch.empty(B, S, 0, dtype=torch.float32, device=index_q.device)
     return ops.prefill_logits(index_q, index_k, weights)
 
@@ -208,7 +216,10 @@ def dense_mla_core(q: torch.Tensor, kv: torch.Tensor, value_dim: int,
     B, S, H, _ = q.shape
     if sm_scale is None:
         sm_scale = q.shape[-1] ** -0.5
-    if kv.shape[1] == 0:  # no key: every row is empty
+    if kv.shape[1] == 0:  # no key: every row is empty, the other limits hold
+        _need_rows(B * S)
+        if not 16 <= H <= 1024:
+            raise RuntimeError(f"the head count must be 16 to 1024 (got {H})")
         return torch.zeros(B, S, H, LATENT_DIM, dtype=q.dtype, device=q.device)
     out = ops.prefill_attention(q.to(torch.bfloat16).contiguous(), kv, sm_scale=float(sm_scale))
     return out.to(q.dtype)

@@ -66,3 +66,27 @@ def test_accepted(dev):
     bits = ops.selection_set(a["idx"], 40, True)
     assert ops.selection_set(a["idx"].int(), 40, False).shape == (6, 8)
     assert ops.prefill_attention(a["q"], a["kv"], bits).shape == (2, 3, 16, 512)
+
+
+def test_empty_contexts(dev):
+    """No key: empty scores and zero rows, for the shapes that a context of
+    one key is taken with, and refused like it for the others."""
+    from lagged_indexer_dsa_amd import attention_core as ac
+
+    for T in (0, 1):
+        def logits(B, S, H):
+            return ac.indexer_logits(torch.zeros(B, S, H, 128, device=dev), torch.zeros(B, T, 128, device=dev),
+                                     torch.zeros(B, S, H, device=dev))
+
+        def dense(B, S, H):
+            return ac.dense_mla_core(torch.ones(B, S, H, 576, dtype=torch.bfloat16, device=dev),
+                                     torch.zeros(B, T, 576, dtype=torch.bfloat16, device=dev), 512)
+
+        assert logits(2, 3, 32).shape == (2, 3, T)
+        assert dense(2, 3, 32).shape == (2, 3, 32, 512) and not dense(2, 3, 32).any()
+        for shape in ((2, 3, 24), (2, 3, 80), (2, 0, 32), (1, 65536, 16)):
+            with pytest.raises(RuntimeError):
+                logits(*shape)
+        for shape in ((1, 1, 1040), (1, 2, 0), (2, 0, 32), (1, 65536, 16)):
+            with pytest.raises(RuntimeError):
+                dense(*shape)
