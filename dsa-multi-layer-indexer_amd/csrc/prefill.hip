@@ -35,8 +35,10 @@ static_assert(kPfLoads * kPfThreads == kPfKeys * kPfRowChunks, "whole loads");
 
 constexpr float kPfRise = 32.f;
 // A wave takes the second bf16 term of a tile's probabilities too when one of
-// its rows has a probability above this share of the row's sum so far.
+// its rows has a probability above this share of the row's sum so far; with
+// fewer keys a split than kPfBothKeys it always does.
 constexpr float kPfSecond = 1.f / 24.f;
+constexpr int kPfBothKeys = 512;
 
 struct PrefillArgs {
   const uint16_t* q;     // [B, S*H, 576] bf16
@@ -104,7 +106,7 @@ __device__ __forceinline__ float half_swap_sum(float v) {
 // a decode row per query took 1115 us and 2.5 ms of workspace fills.
 // Fragments read 4, 6, 8 and 10 steps ahead, with one term: 193, 184, 182 and
 // 210 us of kernel.
-template <bool MASK>
+template <bool MASK, bool BOTH>
 __global__ __launch_bounds__(kPfThreads, 1) void prefill_attention_kernel(const PrefillArgs A) {
   __shared__ __align__(16) uint16_t kb[2 * kPfKeys * DSA_QK_DIM];
   __shared__ int redo;
@@ -265,28 +267,48 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_attention_kernel(const 
     //   1024 over 4096, masked  0.00198 170  .00192 189  .00188 198  .00184 204  .00166 204
     // (a decode row a query, rounded about its running maximum: 0.00196,
     // 0.00192, 0.00172 and 0.00194).
-    const bool two = __ballot(__builtin_amdgcn_exp2f(tmax - mr) > kPfSecond * half_swap_sum(l)) != 0;  // uniform
-    // one copy of the products in the code: unrolled, or as two branches, the
-    // accumulators cross the vector file at the join and spill
-#pragma nounroll
-    for (int term = 0;; ++term) {
-      uint4 vf[kPfDepth];
+    // what the rounding left of the probabilities, and its sum
+    const auto second = [&](uint32_t* w) {
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) {
+        w[i >> 1] = pack_bf16x2(s[0][i] - __uint_as_float(pk[i >> 1] << 16),
+                                s[0][i + 1] - __uint_as_float(pk[i >> 1] & 0xffff0000u));
+        l = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, w[i >> 1]), __builtin_bit_cast(v2bf, 0x3f803f80u),
+                                            l, false);
+      }
+    };
+    const auto product = [&](const uint4& v, const uint32_t* p, int i) {
+      const uint32_t* pr = p + 4 * (i >> 4);
+      o[i & 15] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(v), as_bf8(make_uint4(pr[0], pr[1], pr[2], pr[3])),
+                                                          o[i & 15], 0, 0, 0);
+    };
+    uint4 vf[kPfDepth];
+    if constexpr (BOTH) {
+      uint32_t pl[8];
+      second(pl);
 #pragma unroll
       for (int i = 0; i < kPfDepth; ++i) vf[i] = v_frag(i);
 #pragma unroll
       for (int i = 0; i < 32; ++i) {
-        const uint32_t* pr = &pk[4 * (i >> 4)];
-        const v8bf pb = as_bf8(make_uint4(pr[0], pr[1], pr[2], pr[3]));
-        o[i & 15] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf8(vf[i % kPfDepth]), pb, o[i & 15], 0, 0, 0);
+        product(vf[i % kPfDepth], pk, i);
+        product(vf[i % kPfDepth], pl, i);
         if (i + kPfDepth < 32) vf[i % kPfDepth] = v_frag(i + kPfDepth);
       }
-      if (term || !two) break;
+    } else {
+      const bool two = __ballot(__builtin_amdgcn_exp2f(tmax - mr) > kPfSecond * half_swap_sum(l)) != 0;  // uniform
+      // one copy of the products in the code: unrolled, or as two branches, the
+      // accumulators cross the vector file at the join and spill
+#pragma nounroll
+      for (int term = 0;; ++term) {
 #pragma unroll
-      for (int i = 0; i < 16; i += 2) {
-        pk[i >> 1] = pack_bf16x2(s[0][i] - __uint_as_float(pk[i >> 1] << 16),
-                                 s[0][i + 1] - __uint_as_float(pk[i >> 1] & 0xffff0000u));
-        l = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, pk[i >> 1]), __builtin_bit_cast(v2bf, 0x3f803f80u),
-                                            l, false);
+        for (int i = 0; i < kPfDepth; ++i) vf[i] = v_frag(i);
+#pragma unroll
+        for (int i = 0; i < 32; ++i) {
+          product(vf[i % kPfDepth], pk, i);
+          if (i + kPfDepth < 32) vf[i % kPfDepth] = v_frag(i + kPfDepth);
+        }
+        if (term || !two) break;
+        second(pk);
       }
     }
   };
@@ -618,8 +640,19 @@ hipError_t launch_prefill_attention(const void* q, const void* keys, const uint3
   A.part_ml = A.part_o + (size_t)A.nsplit * rows * DSA_LATENT_DIM;
   A.sm_log2 = sm_scale * 1.4426950408889634f;
   const dim3 grid((unsigned)((long)A.tiles * A.nsplit * B)), block(kPfThreads);
-  if (mask) hipLaunchKernelGGL(prefill_attention_kernel<true>, grid, block, 0, s, A);
-  else hipLaunchKernelGGL(prefill_attention_kernel<false>, grid, block, 0, s, A);
+  // Short key ranges, where most tiles need the second term: always, read
+  // once.  (us, always and by need: 300 queries and keys, 75 keys a split,
+  // 40.7 and 42.1; 700, 175 keys, 74.1 and 77.2; 1024 over 1200 masked, 344
+  // keys, 87.8 and 92.9; 256 over 3000 masked, 32 heads, 718 keys, 103.7 and
+  // 105.5; 1500 queries and keys of 32 heads, 750 keys, 189 and 176; 512 over
+  // 5000 masked, 1186 keys, 142 and 140; 1024 over 4096 masked, 1792 keys, 205
+  // and 192.)
+  const bool both = (T - std::min(S, T) / 2) / A.nsplit < kPfBothKeys;
+  const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, A); };
+  if (mask && both) go(prefill_attention_kernel<true, true>);
+  else if (mask) go(prefill_attention_kernel<true, false>);
+  else if (both) go(prefill_attention_kernel<false, true>);
+  else go(prefill_attention_kernel<false, false>);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && A.nsplit > 1) {
     hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)rows), block, 0, s, A);

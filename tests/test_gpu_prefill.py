@@ -222,3 +222,29 @@ def test_selection_set_at_the_longest_context(dev, T, itype):
         want = sorted(v for v in {0, T - 1, T - 2, T - 3, T - 4, T // 2, 31, 32} if v < T - S + s + 1)
         assert np.flatnonzero(np.unpackbits(bits[s].view(np.uint8), bitorder="little")).tolist() == want
         assert slots[s].tolist() == want + [-1] * (idx.shape[2] - len(want))
+
+
+@pytest.mark.parametrize("T", [575, 576, 577, 900])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("rising", [False, True])
+def test_second_terms_by_rule_and_by_need(dev, T, masked, rising):
+    """130 row tiles, one split: on both sides of the 512 keys from which the
+    probabilities' second terms are taken by need; also with rows that are
+    redone from their true maximum."""
+    from lagged_indexer_dsa_amd import ops
+
+    print(f"[prefill] second terms T={T} masked={masked} rising={rising}", flush=True)
+    S, H = 130, 128
+    g = torch.Generator(device=dev).manual_seed(T)
+    q = torch.randn(1, S, H, 576, generator=g, device=dev).to(torch.bfloat16)
+    kv = torch.randn(1, T, 576, generator=g, device=dev).to(torch.bfloat16)
+    if rising:
+        kv *= 0.1
+        kv[0, T - 40:T - 30] += q[0, S - 9, 7] * 2.0
+        kv[0, 300] += q[0, 5, 100]
+    mask, bits = _causal(S, T, dev), None
+    if masked:
+        idx = torch.randint(0, T, (1, S, 700), generator=g, device=dev)
+        bits = ops.selection_set(idx, T, True)
+        mask = mask & torch.zeros(1, S, T, dtype=torch.bool, device=dev).scatter_(2, idx, True)[0]
+    _check(ops.prefill_attention(q, kv, bits), q, kv, mask[None])
