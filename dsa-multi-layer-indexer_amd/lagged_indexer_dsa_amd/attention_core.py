@@ -66,17 +66,18 @@ def indexer_logits(index_q: torch.Tensor, index_k: torch.Tensor, weights: torch.
     ``[B, S, H_idx]``; H_idx one of 16, 32, 48, 64.  No causal masking
     (apply it with :func:`apply_causal_mask`, as the reference does).
     """
-    if index_q.dim() != 4:
-        raise ValueError(f"index_q must be [B,S,H,D], got {tuple(index_q.shape)}")
-    if index_k.dim() != 3:
-        raise ValueError(f"index_k must be [B,S_kv,D], got {tuple(index_k.shape)}")
-    B, S, H, D = index_q.shape
-    if index_k.shape[0] != B or index_k.shape[2] != D or tuple(weights.shape) != (B, S, H):
+    qs, ks = index_q.shape, index_k.shape
+    if len(qs) != 4:
+        raise ValueError(f"index_q must be [B,S,H,D], got {tuple(qs)}")
+    if len(ks) != 3:
+        raise ValueError(f"index_k must be [B,S_kv,D], got {tuple(ks)}")
+    B, S, H, D = qs
+    if ks[0] != B or ks[2] != D or weights.shape != qs[:3]:
         raise ValueError("index_q, index_k and weights disagree in B, S, H or D")
     if D != INDEX_DIM:
         raise ValueError(f"the fp8 indexer contracts D = {INDEX_DIM}, got {D}")
     _gpu(index_q, index_k, weights)
-    if index_k.shape[1] == 0:  # no key: nothing to launch, the other limits hold
+    if ks[1] == 0:  # no key: nothing to launch, the other limits hold
         _need_rows(B * S)
         if H not in (16, 32, 48, 64):
             raise RuntimeError(f"index_n_heads must be 16, 32, 48 or 64 (got {H})")

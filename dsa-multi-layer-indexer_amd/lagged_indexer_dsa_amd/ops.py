@@ -24,7 +24,7 @@ from ._lib import (
 
 def _dev(*tensors: torch.Tensor) -> None:
     for t in tensors:
-        if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
+        if not isinstance(t, torch.Tensor) or not t.is_cuda:
             raise RuntimeError("lagged_indexer_dsa_amd ops need GPU (HIP) tensors; there is no CPU path")
         if not t.is_contiguous():
             raise RuntimeError("lagged_indexer_dsa_amd ops need contiguous tensors")
@@ -132,9 +132,10 @@ def select_rows(scores: torch.Tensor, k: int, pad_value: int) -> torch.Tensor | 
     """:func:`topk` with sorted=True over whole rows, as int64 and in one
     launch; None for the shapes the row kernel does not take."""
     _dev(scores)
-    if scores.dim() != 2 or scores.dtype != torch.float32:
+    shape = scores.shape
+    if len(shape) != 2 or scores.dtype != torch.float32:
         raise RuntimeError("scores must be [B, slab] float32")
-    B, slab = scores.shape
+    B, slab = shape
     if not _lib.load().dsa_select_rows_supported(B, slab, k):
         return None
     out = torch.empty(B, k, dtype=torch.int64, device=scores.device)
@@ -257,8 +258,9 @@ def _kernel_input(x: torch.Tensor) -> torch.Tensor:
 
 
 def _need_kv(kv: torch.Tensor) -> None:
-    if kv.dim() != 3 or kv.shape[2] != QK_DIM:
-        raise RuntimeError(f"kv must be [B, T, 576], got {tuple(kv.shape)}")
+    shape = kv.shape
+    if len(shape) != 3 or shape[2] != QK_DIM:
+        raise RuntimeError(f"kv must be [B, T, 576], got {tuple(shape)}")
 
 
 def _pack_source(kv: torch.Tensor) -> torch.Tensor:
@@ -275,14 +277,15 @@ def prefill_logits(q: torch.Tensor, k: torch.Tensor, w: torch.Tensor) -> torch.T
     k [B, T, 128], quantised per row inside.  Reference: attention_core.py:27-49."""
     q, k, w = _kernel_input(q), _kernel_input(k), _kernel_input(w)
     _dev(q, k, w)
-    if q.dim() != 4 or q.shape[3] != INDEX_DIM:
-        raise RuntimeError(f"q must be [B, S, H, 128], got {tuple(q.shape)}")
-    B, S, H, _ = q.shape
-    if k.dim() != 3 or k.shape[0] != B or k.shape[2] != INDEX_DIM:
-        raise RuntimeError(f"k must be [{B}, T, 128], got {tuple(k.shape)}")
-    if w.shape != (B, S, H):
+    qs, ks = q.shape, k.shape  # (each read of a shape builds it anew)
+    if len(qs) != 4 or qs[3] != INDEX_DIM:
+        raise RuntimeError(f"q must be [B, S, H, 128], got {tuple(qs)}")
+    B, S, H, _ = qs
+    if len(ks) != 3 or ks[0] != B or ks[2] != INDEX_DIM:
+        raise RuntimeError(f"k must be [{B}, T, 128], got {tuple(ks)}")
+    if w.shape != qs[:3]:
         raise RuntimeError(f"w must be {(B, S, H)}, got {tuple(w.shape)}")
-    T = k.shape[1]
+    T = ks[1]
     ws = torch.empty(_lib.load().dsa_prefill_logits_workspace_bytes(B, S, H, T), dtype=torch.uint8, device=q.device)
     out = torch.empty(B, S, T, dtype=torch.float32, device=q.device)
     _lib.call("dsa_prefill_logits", q.data_ptr(), _PACK_DTYPES[q.dtype], k.data_ptr(), _PACK_DTYPES[k.dtype],
@@ -311,9 +314,10 @@ def selection_set(idx: torch.Tensor, T: int, as_bits: bool) -> torch.Tensor:
     row, or the KV slots b * T + position ascending, then -1 [B * S, n]."""
     idx = idx.contiguous()
     _dev(idx)
-    if idx.dim() != 3 or idx.dtype not in (torch.int32, torch.int64):
-        raise RuntimeError(f"idx must be [B, S, n] int32 or int64, got {idx.dtype} {tuple(idx.shape)}")
-    B, S, n = idx.shape
+    shape = idx.shape
+    if len(shape) != 3 or idx.dtype not in (torch.int32, torch.int64):
+        raise RuntimeError(f"idx must be [B, S, n] int32 or int64, got {idx.dtype} {tuple(shape)}")
+    B, S, n = shape
     lib = _lib.load()
     if as_bits:
         out = torch.empty(lib.dsa_selection_bits_bytes(B * S, T) // 4, dtype=torch.int32, device=idx.device)
@@ -332,12 +336,13 @@ def prefill_attention(q: torch.Tensor, kv: torch.Tensor, bits: torch.Tensor | No
     _need_kv(kv)
     kv = _pack_source(kv)
     _dev(q, kv)
-    if q.dim() != 4 or q.shape[3] != QK_DIM or q.dtype != torch.bfloat16:
+    qs = q.shape
+    if len(qs) != 4 or qs[3] != QK_DIM or q.dtype != torch.bfloat16:
         raise RuntimeError("q must be [B, S, H, 576] bfloat16")
-    B, S, H, _ = q.shape
-    if kv.shape[0] != B:
-        raise RuntimeError(f"kv holds {kv.shape[0]} requests, q {B}")
-    T = kv.shape[1]
+    B, S, H, _ = qs
+    requests, T, _ = kv.shape
+    if requests != B:
+        raise RuntimeError(f"kv holds {requests} requests, q {B}")
     lib = _lib.load()
     keys = torch.empty(lib.dsa_prefill_keys_bytes(B, T), dtype=torch.uint8, device=q.device)
     ws = torch.empty(lib.dsa_prefill_workspace_bytes(B, S, H, T), dtype=torch.uint8, device=q.device)
