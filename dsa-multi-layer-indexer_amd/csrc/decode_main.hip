@@ -1885,12 +1885,17 @@ __global__ __launch_bounds__(kMainThreads, (ROLES & ~kRolePlan) == kRoleScan ? 4
 // and of the rest its share of all keys (at most one for 64 keys, and
 // kMaxSplit; the products stay below 2^32: W < 256, u <= 2^24).  A.nsplit
 // splits of every row's capacity leave the workgroups of short rows idle:
-// rows of 777, 20000 and 32768 keys x 64 heads took 59.5 us, the longest
-// one's splits holding 1561 keys; now 850, and 44.4.  Eight rows of 500 to
-// 16000 keys x 64 heads: 69.5 -> 39.3; 30 rows of 2000 keys in a table of
-// the same size 48 -> 42.5 (spare workgroups used); rows of equal length
-// that fill their tables keep their splits and pay for the lengths being
-// read first: 4 x 5000 keys 15.2 -> 15.5, 2 x 131072 keys 50.4 -> 50.9.
+// rows of 777, 20000 and 32768 keys x 64 heads took 59.2 us, the longest
+// one's splits holding 1561 keys; now 850, and 44.1.  Rows of 8537, 24822 and
+// 32768 keys x 64 heads: 61.8 -> 51.9.  Eight rows of 500 to 16000 keys x 64
+// heads: 69.3 -> 43.8; 30 rows of 2000 keys x 64 heads 47.8 -> 42.2 (spare
+// workgroups used).  Rows of equal length that fill their tables keep their
+// splits and pay for the lengths being read first: 4 x 5000 keys 14.1 -> 14.6,
+// 2 x 131072 keys 57.8 -> 58.7 (calls over rotated inputs; the length of the
+// row taken from the lanes instead of read again, or the page table's entries
+// fetched ahead for equal rows, change that by less than 0.2).
+// A row's split points, and so the last bits of its sums, follow from the
+// lengths of all rows in the call.
 // What bounds it now is the 128-key tile, ~4 us, times the tiles a split
 // holds.  A head group's workgroups are contiguous in the grid, as the other
 // launches' splits of a (row, head group) are.

@@ -1,6 +1,6 @@
 // Sparse / dense MLA decode of many rows (gfx950): one workgroup takes all the
-// keys of a (row, head group).  The operation is the decode launch's attention
-// (decode_main.hip):
+// keys of a (row, head group).  For calls of the attention alone; in a decode
+// layer it stays the decode launch's (decode_main.hip), whose operation it is:
 //   out[b,h,:] = sum_j softmax_j(sm * q[b,h,:] . kv_j) * kv_j[:512],
 //   kv_j = bf16_rn(f32(e4m3) * scale[d/128]) | bf16 rope.
 //

@@ -101,7 +101,7 @@ __device__ __forceinline__ float half_swap_sum(float v) {
 // flight while this one is used.
 //
 // Bound by the matrix cores and the LDS reads that feed them: a call with 2999
-// causal queries of 16 heads takes 220 us (156 GFLOP and the second terms of
+// causal queries of 16 heads takes 209-220 us by card (156 GFLOP and the second terms of
 // the probabilities; a library product of 8192^3 reaches 1218 TFLOP/s here);
 // a decode row per query took 1115 us and 2.5 ms of workspace fills.
 // Fragments read 4, 6, 8 and 10 steps ahead, with one term: 193, 184, 182 and

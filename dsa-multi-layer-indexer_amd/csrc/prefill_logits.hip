@@ -15,7 +15,7 @@
 // and 57 ns per 4 MFMAs and 32 VALU operations with four waves a SIMD,
 // together 81): 1024 rows x 8192 keys x 64 heads in 65 us (2.1
 // PFLOP/s of fp8) where the decode scan's flat form took 146 and torch's
-// quantisation and page layout 200 before it; here that is 10 (two launches).
+// quantisation and page layout 200 before it; here that is 14 (two launches).
 // Neither 128 keys a wave, nor the products of the next head group issued
 // before this group's sums, nor wave priorities around them moved it by more
 // than 3%.

@@ -23,11 +23,12 @@
 // equal scores, or a range set by an outlier) takes the general form: t* by
 // radix digits, then a bitonic sort.
 //
-// Bound by the latency of these steps, four rows a CU in flight.  1024 rows of
-// 8192 scores, top-2048: 33 us (1.5 TB/s of scores and int64 indices), where
-// the slice kernels took 793 (their finalize keeps one row per CU: 150 KB of
-// LDS, and sorts it with a barrier a stage); 16384 scores 76, 2048 scores 16;
-// with every bin crowded (ties) 158.
+// Bound by the latency of these steps, three rows a CU in flight (78 registers
+// for rows of 4097 to 8192 scores: six waves a SIMD).
+// 1024 rows of 8192 scores, top-2048: 32 us (1.6 TB/s of scores and int64
+// indices), where the slice kernels took 793 (their finalize keeps one row per
+// CU: 150 KB of LDS, and sorts it with a barrier a stage); 16384 scores 76, 2048
+// scores 16; with every bin crowded (ties) 158.
 #include "dsa_common.h"
 #include "dsa_kernels.h"
 

@@ -8,8 +8,7 @@
 // topk_selector.py:36-194; in-kernel exact select K:1097-1129, K:1248-1310).
 //
 // The sorted select of many rows, or of rows up to 131072 scores, is
-// select_rows.hip's; this file's form is for a few longer rows and top-k
-// above its limit.
+// select_rows.hip's; this file's sorted form is for fewer than 24 longer rows.
 //
 // Two launches (the histogram is fused into the indexer scan on the decode
 // path, leaving one), so a 128K-196K row is read by many CUs:

@@ -211,7 +211,9 @@ int dsa_sparse_mla_decode(const void* q_bf16, const void* kv_pool,
  * (seq_lens clamped to pt_stride*64).  workspace:
  * dsa_sparse_mla_workspace_bytes(B, H, nsplit), as for (3); nsplit = 0:
  * one split per 64 keys of the page table's capacity, at most 128.  From 2 to
- * 64 rows whose splits are all resident share B * nsplit splits by length.
+ * 64 rows whose splits are all resident share B * nsplit splits by length:
+ * where a row's keys are divided, and so the last bits of its output, then
+ * depends on the other rows' lengths (the same call always gives the same).
  * Replaces: dense_mla_core (attention_core.py:142-160), the full-attention
  * layers and the DENSE cold start of DSAModel.forward (model.py:51-59,
  * 104-114).
