@@ -59,3 +59,11 @@ def test_dense_rows_by_length(dev, lens, H, extra, nsplit):
         bound = 1.01 * 2.0 ** -8 * (w @ k[:, :512].abs() + ref.abs())
         bad = (outs[0][b].double() - ref).abs() > bound + 1e-30
         assert not bad.any(), f"row {b}: {int(bad.sum())} off"
+
+
+@pytest.mark.parametrize("lens,H,extra", [([2000], 16, 2016), ([2000], 64, 2016), ([1], 16, 2047), ([0], 16, 2048),
+                                          ([2000, 2000], 16, 2016), ([65, 1, 4000], 64, 1985)])
+def test_rows_in_a_table_of_131072_keys(dev, lens, H, extra):
+    """One row keeps the even division of the table, whose later splits hold
+    no key; several share the splits by length."""
+    test_dense_rows_by_length(dev, lens, H, extra, 0)
